@@ -183,12 +183,14 @@ typedef struct tms_sample_args {
                                  every row is greedy or has 1 <= top_k <= 128, and
                                  the library may take its top-k kernel (it does when
                                  batch x chunks <= 1024 workgroups).  Every other
-                                 call takes the general kernel, whose row mergers
-                                 sample whole any row the candidate lists cannot
-                                 finish (top-p rows with more than 1024 entries
-                                 within 40 of the maximum, draws past those
-                                 entries, rows that break the promise) in the same
-                                 launch.  In the top-k kernel a row that breaks the
+                                 call takes the general kernel.  Rows that its
+                                 candidate lists cannot finish (top-p rows with more
+                                 than 1024 entries within 40 of the maximum, draws
+                                 past those entries) are sampled by the
+                                 whole-vocabulary kernel, a second launch of every
+                                 call without the promise (vocab <= 262144); with it,
+                                 and without a context, by the row's merger in the
+                                 same launch, more slowly.  In the top-k kernel a row that breaks the
                                  promise gets TMS_ROW_UNSUPPORTED, never a wrong
                                  sample */
     uint32_t reserved;        /* must be 0 */
@@ -267,7 +269,8 @@ int tms_workspace_reset(tms_context* ctx, hipStream_t stream);
 
 /*
  * Batched mask -> penalties -> temperature -> top-k -> softmax -> top-p /
- * min-p -> draw, one launch, stream-ordered, no host synchronisation.
+ * min-p -> draw, one launch (two without the top-k promise, for rows that
+ * need the whole vocabulary), stream-ordered, no host synchronisation.
  * Replaces sample_token (tensormark/llama_chat.cpp:146-153) with the grammar
  * restriction of tensormark/llama_chat.cpp:184-209, i.e. the composition of
  * apply_repeat_penalty (tensormark/tmsample.h:52-63) and tmsample::sample

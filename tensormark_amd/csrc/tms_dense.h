@@ -1,12 +1,13 @@
 // tms_dense.h -- the exact full-row form of tmsample::sample
-// (tensormark/tmsample.h:177-200) for the rows the general kernel cannot
-// finish from its candidate lists: top-p rows (top_k = 0 or large) whose
+// (tensormark/tmsample.h:177-200), for what tms_topp.hip does not decide and,
+// in calls without that kernel, for the rows the general kernel cannot finish
+// from its candidate lists: top-p rows (top_k = 0 or large) whose
 // significant entries (v / T within 40 of the maximum) outnumber the list
 // capacity, a draw that lands past the last significant entry, id lists
 // longer than the held entries.
 //
-// The row's merger samples such a row itself, right where it finds it needs
-// the whole row (no second launch): 256 threads of its workgroup, over a
+// The row's workgroup samples such a row itself, right where it finds it
+// needs the whole row: 256 of its threads, over a
 // region of the context's workspace (2 x vocab 64-bit words) taken by a
 // lock (dense_inline):
 //

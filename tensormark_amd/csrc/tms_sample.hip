@@ -1,6 +1,7 @@
 // tms_sample.hip -- batched token sampler for gfx950 (MI355X).
 //
-// One launch per call.  Row b of the batch is cut into S chunks of at most
+// One launch per call, and for calls without the top-k promise a second that
+// samples the dense top-p rows (tms_topp.hip).  Row b of the batch is cut into S chunks of at most
 // 16K ids; workgroup (b, c) streams its chunk from HBM once with 16-byte
 // loads into registers (64 values per thread), applies the grammar mask and
 // the history penalties there, and reduces the chunk to a short sorted
@@ -20,7 +21,8 @@
 //   top-p   K > kTopkFast (top_k = 0 or large): every chunk entry whose
 //           probability can change the fp64 sums, i.e. v / T within 40 of
 //           the chunk maximum (exp(-40) < 2^-57); rows past the capacity
-//           are sampled whole by their merger (tms_dense.h).
+//           are left to the whole-vocabulary kernel (QUEUE), or sampled
+//           whole by their merger (tms_dense.h).
 //
 // Timeline of a workgroup: the stream's loads are the kernel's first
 // instructions and are issued unconditionally (clamped addresses, an all-ones
@@ -43,6 +45,7 @@
 
 #include "tms_dense.h"
 #include "tms_select.h"
+#include "tms_topp.h"
 
 namespace tms {
 
@@ -89,7 +92,13 @@ __device__ __forceinline__ int stage_log2(int S) {
 // window on 16-byte-aligned 2-byte rows, whose stream stays in registers as
 // the masked raw vectors (half the registers of widened values), so a
 // chunk holds 20480 ids and fewer workgroups cover a row.
-template <typename T, bool FAST, int NV>
+//
+// QUEUE: a dense top-p row is left to the whole-vocabulary kernel that the
+// call launches next (tms_topp.hip); its merger marks the row.  Otherwise the
+// merger samples it whole in place (dense_inline), for calls that promise
+// top-k rows, where a second launch would cost every call for rows that break
+// the promise.
+template <typename T, bool FAST, int NV, bool QUEUE>
 __global__ __launch_bounds__(kBlock, 3) void sample_kernel(KArgs a) {
     constexpr int VEC = Elt<T>::kVec;
     constexpr int NVT = NV / VEC;
@@ -470,7 +479,24 @@ __global__ __launch_bounds__(kBlock, 3) void sample_kernel(KArgs a) {
         }
         TMS_TR(20);
         int n = 0;
-        if (!anynf && !bad_params && !fallback) {
+        bool crowded = false;
+        if constexpr (QUEUE) {
+            if (mode == MODE_TOPP) {
+                // More slots reach thr than the list holds entries: the row is
+                // left to the next launch, and nothing is staged.
+                int hot = 0;
+#pragma unroll
+                for (int j = 0; j < NVT; ++j) hot += __popcll(__ballot(vmax[j] >= thr));
+                if (lane == 0) sm.list_src[wv] = hot;
+                lds_sync();
+                hot = 0;
+#pragma unroll
+                for (int w = 0; w < kWaves; ++w) hot += sm.list_src[w];
+                crowded = hot > kCand;
+                if (crowded) n = kCand + 1;
+            }
+        }
+        if (!anynf && !bad_params && !fallback && !crowded) {
             // Each wave compacts its candidates with ballots into its own
             // segment of cand (kCand / kWaves entries), as raw (value, id).
             constexpr int kSeg = kCand / kWaves;
@@ -770,6 +796,11 @@ __global__ __launch_bounds__(kBlock, 3) void sample_kernel(KArgs a) {
     // lists merged.
     if (t == 64) st_agent(&a.counters[row * kCounterStride], 0u);   // ready for the next launch (wave 0 keeps no store in flight)
     uint64_t* uni = sm.big.m.uni;
+    if constexpr (QUEUE) {
+        // the row's state (below TOPP_NONE unless the row is left to the next
+        // launch) and its workgroups' shared words
+        if (t < kToppCtl) a.topp_ctl[row * kToppCtl + t] = 0u;
+    }
     if (t == 0) {
         sm.theta = 0;     // lists to read again (bit per list)
         sm.misc[3] = 0;   // a list never arrived
@@ -1184,7 +1215,12 @@ __global__ __launch_bounds__(kBlock, 3) void sample_kernel(KArgs a) {
         lds_sync();
         whole = sm.nvalid != 0;
     }
-    if (__builtin_expect(whole, 0)) {
+    if constexpr (QUEUE) {
+        if (whole && t == 0) {
+            a.topp_ctl[row * kToppCtl] = go_dense ? TOPP_SELECT : TOPP_WHOLE;
+            *a.topp_any = a.topp_call;
+        }
+    } else if (__builtin_expect(whole, 0)) {
         [[clang::always_inline]] dense_inline<T>(a, row, *reinterpret_cast<DenseLds*>(&sm.big));
     }
 }
@@ -1214,6 +1250,41 @@ extern "C" const char* tms_status_string(int code) {
         case TMS_ERR_NO_DEVICE: return "no HIP device";
         default: return "unknown";
     }
+}
+
+// The general kernel for this call's type and alignment: QUEUE, then the
+// whole-vocabulary kernel, when the call has its workspace (tms_topp.h).
+template <typename T, int NV>
+static void launch_general_t(const tms::KArgs& k, bool fast, int batch, hipStream_t stream) {
+    const dim3 grid((unsigned)(batch * k.S)), block(tms::kBlock);
+    const bool queue = k.hist != nullptr;
+    if constexpr (NV != tms::kEpt) {   // the packed stream: aligned rows
+        if (queue) hipLaunchKernelGGL((tms::sample_kernel<T, true, NV, true>), grid, block, 0, stream, k);
+        else hipLaunchKernelGGL((tms::sample_kernel<T, true, NV, false>), grid, block, 0, stream, k);
+    } else if (fast) {
+        if (queue) hipLaunchKernelGGL((tms::sample_kernel<T, true, NV, true>), grid, block, 0, stream, k);
+        else hipLaunchKernelGGL((tms::sample_kernel<T, true, NV, false>), grid, block, 0, stream, k);
+    } else {
+        if (queue) hipLaunchKernelGGL((tms::sample_kernel<T, false, NV, true>), grid, block, 0, stream, k);
+        else hipLaunchKernelGGL((tms::sample_kernel<T, false, NV, false>), grid, block, 0, stream, k);
+    }
+}
+
+static int launch_general(const tms::KArgs& k, int dtype, bool fast, bool packed, int batch, int cus,
+                          hipStream_t stream) {
+    switch (dtype) {
+        case TMS_DTYPE_F32: launch_general_t<float, tms::kEpt>(k, fast, batch, stream); break;
+        case TMS_DTYPE_F16:
+            if (packed) launch_general_t<_Float16, tms::kEptPacked>(k, fast, batch, stream);
+            else launch_general_t<_Float16, tms::kEpt>(k, fast, batch, stream);
+            break;
+        default:
+            if (packed) launch_general_t<tms::Bf16, tms::kEptPacked>(k, fast, batch, stream);
+            else launch_general_t<tms::Bf16, tms::kEpt>(k, fast, batch, stream);
+            break;
+    }
+    if (k.hist) return tms_launch_topp(k, dtype, batch, cus, stream);
+    return hipGetLastError() == hipSuccess ? TMS_OK : TMS_ERR_HIP;
 }
 
 static int chunks_for(int V) { return (V + tms::kChunk - 1) / tms::kChunk; }
@@ -1257,7 +1328,15 @@ extern "C" int tms_create(int device, int max_batch, int max_vocab, tms_context*
     // The whole-row path's region: never read before it is written, so not
     // cleared.
     ctx->dense_slots = std::min(max_batch, tms::kDenseSlotsMax);
-    ctx->dense_bytes = (size_t)ctx->dense_slots * 2 * (size_t)max_vocab * sizeof(uint64_t);
+    // With it, the second launch's records (tms_topp.h), likewise written
+    // before they are read.
+    const size_t dense_words = (size_t)ctx->dense_slots * 2 * (size_t)max_vocab;
+    const size_t hist_words = tms::topp_hist_words(nb, max_vocab);
+    const size_t item_words = nb * tms::kToppRanges * tms::kToppItemWords;
+    const size_t off_hw = (dense_words + 31) / 32 * 32;
+    const size_t off_iw = off_hw + hist_words;
+    const size_t off_cw = off_iw + item_words;
+    ctx->dense_bytes = (off_cw + nb * tms::kToppCtl / 2 + 32) * sizeof(uint64_t);
     if (rc == TMS_OK && hipMalloc(&ctx->dense, ctx->dense_bytes) != hipSuccess) {
         ctx->dense = nullptr;
         rc = TMS_ERR_HIP;
@@ -1280,6 +1359,11 @@ extern "C" int tms_create(int device, int max_batch, int max_vocab, tms_context*
     ctx->ov_n = (int32_t*)(p + off_hn);
     ctx->ov_ids = (int32_t*)(p + off_hi);
     ctx->ov_vals = (float*)(p + off_hv);
+    ctx->hist = ctx->dense + off_hw;
+    ctx->topp_items = ctx->dense + off_iw;
+    ctx->topp_ctl = (uint32_t*)(ctx->dense + off_cw);
+    ctx->topp_any = ctx->topp_ctl + nb * tms::kToppCtl;
+    ctx->topp_calls = 0;
     ctx->ones_begin = off_ones;
     ctx->ones_end = off_l;
     (void)hipSetDevice(prev);
@@ -1340,6 +1424,11 @@ struct SampleWs {
     int32_t* ov_n;         // the history pre-pass's lists
     int32_t* ov_ids;
     float* ov_vals;
+    uint64_t* hist = nullptr;        // tms_topp.h (contexts only)
+    uint32_t* topp_ctl = nullptr;
+    uint32_t* topp_any = nullptr;
+    uint32_t topp_call = 0;
+    uint64_t* topp_items = nullptr;
 };
 
 // tms_sample_batch over workspace w (a context's, or the allocation-free
@@ -1389,12 +1478,20 @@ static int sample_launch(const SampleWs& w, const tms_sample_args* a, hipStream_
     k.lists = w.lists;
     k.tlists = w.tlists;
     // Any row a chunked kernel cannot finish from its candidate lists is
-    // sampled whole by its own merger, in a region of the workspace taken
-    // by a lock (no second launch).
+    // sampled whole in a region of the workspace taken by a lock, by its own
+    // merger or (QUEUE) by the second launch.
     k.dense = w.dense;
     k.dense_stride = w.max_vocab;
     k.dlocks = w.dlocks;
     k.dense_slots = w.dense_slots;
+    // Calls without the top-k promise: dense top-p rows by a second launch.
+    if (a->row_kinds != TMS_ROWS_TOPK && w.hist && a->vocab <= tms::kToppMaxVocab) {
+        k.hist = w.hist;
+        k.topp_ctl = w.topp_ctl;
+        k.topp_any = w.topp_any;
+        k.topp_call = w.topp_call;
+        k.topp_items = w.topp_items;
+    }
 #ifdef TMS_TRACE
     k.trace = g_tms_trace_host;
 #endif
@@ -1411,24 +1508,7 @@ static int sample_launch(const SampleWs& w, const tms_sample_args* a, hipStream_
         k.recent_stride = tms::kHistMax;
         k.ov_vals = w.ov_vals;
         k.dense = w.dense;
-        const dim3 grid((unsigned)(a->batch * k.S)), block(tms::kBlock);
-#define TMS_LAUNCH(T, F) hipLaunchKernelGGL((tms::sample_kernel<T, F, tms::kEpt>), grid, block, 0, stream, k)
-        switch (a->dtype) {
-            case TMS_DTYPE_F32:
-                if (fast) TMS_LAUNCH(float, true);
-                else TMS_LAUNCH(float, false);
-                break;
-            case TMS_DTYPE_F16:
-                if (fast) TMS_LAUNCH(_Float16, true);
-                else TMS_LAUNCH(_Float16, false);
-                break;
-            default:
-                if (fast) TMS_LAUNCH(tms::Bf16, true);
-                else TMS_LAUNCH(tms::Bf16, false);
-                break;
-        }
-#undef TMS_LAUNCH
-        return hipGetLastError() == hipSuccess ? TMS_OK : TMS_ERR_HIP;
+        return launch_general(k, a->dtype, fast, false, a->batch, device_cus(), stream);
     }
     if (a->row_kinds == TMS_ROWS_SPARSE_MASK && a->mask && a->vocab <= tms::kSparseMaxVocab) {
         // Few allowed ids a row (the caller's hint): one workgroup a row
@@ -1484,28 +1564,7 @@ static int sample_launch(const SampleWs& w, const tms_sample_args* a, hipStream_
         const int per_p = (a->vocab + k.S - 1) / k.S;
         k.CE = (per_p + vec - 1) / vec * vec;
     }
-    const dim3 grid((unsigned)(a->batch * k.S)), block(tms::kBlock);
-#define TMS_LAUNCH(T, F) hipLaunchKernelGGL((tms::sample_kernel<T, F, tms::kEpt>), grid, block, 0, stream, k)
-#define TMS_LAUNCH_PACKED(T) hipLaunchKernelGGL((tms::sample_kernel<T, true, tms::kEptPacked>), grid, block, 0, stream, k)
-    switch (a->dtype) {
-        case TMS_DTYPE_F32:
-            if (fast) TMS_LAUNCH(float, true);
-            else TMS_LAUNCH(float, false);
-            break;
-        case TMS_DTYPE_F16:
-            if (packed) TMS_LAUNCH_PACKED(_Float16);
-            else if (fast) TMS_LAUNCH(_Float16, true);
-            else TMS_LAUNCH(_Float16, false);
-            break;
-        default:
-            if (packed) TMS_LAUNCH_PACKED(tms::Bf16);
-            else if (fast) TMS_LAUNCH(tms::Bf16, true);
-            else TMS_LAUNCH(tms::Bf16, false);
-            break;
-    }
-#undef TMS_LAUNCH_PACKED
-#undef TMS_LAUNCH
-    return hipGetLastError() == hipSuccess ? TMS_OK : TMS_ERR_HIP;
+    return launch_general(k, a->dtype, fast, packed, a->batch, device_cus(), stream);
 }
 
 extern "C" int tms_sample_batch(tms_context* ctx, const tms_sample_args* a, hipStream_t stream) {
@@ -1523,6 +1582,11 @@ extern "C" int tms_sample_batch(tms_context* ctx, const tms_sample_args* a, hipS
     w.ov_n = ctx->ov_n;
     w.ov_ids = ctx->ov_ids;
     w.ov_vals = ctx->ov_vals;
+    w.hist = ctx->hist;
+    w.topp_ctl = ctx->topp_ctl;
+    w.topp_any = ctx->topp_any;
+    w.topp_call = ++ctx->topp_calls;
+    w.topp_items = ctx->topp_items;
     return sample_launch(w, a, stream);
 }
 

@@ -1,0 +1,80 @@
+// tms_topp.h -- the workspace that the general kernel (tms_sample.hip), which
+// marks the dense top-p rows of a call, and the whole-vocabulary kernel
+// (tms_topp.hip), which samples them, share.
+#pragma once
+
+#include "tms_sample_common.h"
+
+namespace tms {
+
+// A record describes one chunk of a row over buckets of lg = penalised value
+// / T, 1/25 wide: each bucket's softmax mass, the number of entries above it,
+// and the chunk's ids in bucket order (a counting sort), so that any interval
+// of buckets is one run of ids a chunk.
+//
+// Buckets run from the one holding the chunk's maximum downwards: 1023 x 1/25
+// spans 40.9, more than kSigSpan, so every entry that can change a sum has
+// one.  At 1/25 a bucket of a 256,000-id normal row holds at most about 1,700
+// entries, so a cut or a draw is settled by ordering a few thousand keys.
+constexpr int kHistBuckets = 1024;
+constexpr float kHistScale = 25.0f;
+constexpr int kHistExtra = 1024;        // penalised entries of a chunk, at most
+constexpr int kHistIds = 16384;         // ids of a chunk, at most: 16 a thread
+constexpr int kHistIdsSmall = 8192;     // ... where that gives more workgroups work
+constexpr int kToppMaxVocab = 262144;
+// u64 words of a record: masses, then u32 counts of the entries above bucket
+// 0..1023, the penalised entries (value bits << 32 | id), the head (valid << 32
+// | bits of the chunk's maximum of lg), and u16 ids in bucket order (below the
+// chunk's length: id - its first id; else kHistIds + the index of a penalised
+// entry).
+constexpr int kHistCnt = kHistBuckets;
+constexpr int kHistExt = kHistCnt + kHistBuckets / 2;
+constexpr int kHistHead = kHistExt + kHistExtra;
+constexpr int kHistId = kHistHead + 2;
+static_assert(kHistIds + kHistExtra < 65536, "16-bit ids of a chunk");
+constexpr int hist_words(int chunk_ids) { return kHistId + chunk_ids / 4 + 2; }
+// Rows in small chunks at most, so that their records fit those of a whole
+// batch in large ones.
+constexpr int kHistSmallRows = 32;
+inline size_t topp_hist_words(size_t rows, int vocab) {
+    const size_t large = rows * (size_t)((vocab + kHistIds - 1) / kHistIds) * hist_words(kHistIds);
+    const size_t few = rows < (size_t)kHistSmallRows ? rows : (size_t)kHistSmallRows;
+    const size_t small = few * (size_t)((vocab + kHistIdsSmall - 1) / kHistIdsSmall) * hist_words(kHistIdsSmall);
+    return (large > small ? large : small) + 32;
+}
+// Row states the general kernel leaves for the whole-vocabulary kernel.
+enum : uint32_t { TOPP_NONE = 0, TOPP_SELECT = 1, TOPP_WHOLE = 2 };
+// u32 words per row shared by the workgroups of a row (zeroed by the general
+// kernel's merger): see tms_topp.hip.
+constexpr int kToppCtl = 64;
+constexpr int kToppRanges = 64;       // most ranges of a row
+constexpr int kToppRawMax = 24;       // raw entries of a range
+constexpr int kToppItemWords = 160;   // u64 words of a range's items: count, then 3 an item
+static_assert(1 + 3 * (2 * kToppRawMax + 1) <= kToppItemWords, "a range's items");
+
+// The bucket of lg, on a grid common to every chunk: floor(25 lg), clamped so
+// that differences of two buckets do not overflow (monotone in lg).
+__device__ __forceinline__ int topp_bucket(float lg) {
+    const float y = fminf(fmaxf(lg * kHistScale, -5e8f), 5e8f);
+    return (int)floorf(y);
+}
+
+// e^x for x in [-42, 0] within 2 ulp (exp64 without its special cases).
+__device__ __forceinline__ double exp_span(double x, const double* tab) {
+    const double kd = rint(x * 0x1.71547652b82fep+6);
+    double r = fma(-kd, 0x1.62e42fefa39efp-7, x);
+    r = fma(-kd, 0x1.abc9e3b39803fp-62, r);
+    double p = 1.0 / 120;
+    p = fma(p, r, 1.0 / 24);
+    p = fma(p, r, 1.0 / 6);
+    p = fma(p, r, 0.5);
+    p = fma(p, r, 1.0);
+    p = fma(p, r, 1.0);
+    const int ki = (int)kd;
+    return ldexp(tab[ki & 63] * p, ki >> 6);
+}
+
+}  // namespace tms
+
+// Launches the whole-vocabulary kernel over `batch` rows (tms_topp.hip).
+int tms_launch_topp(const tms::KArgs& k, int dtype, int batch, int cus, hipStream_t stream);

@@ -1,0 +1,128 @@
+"""GPU parity of the whole-vocabulary kernel (tms_topp.hip): top-p rows with
+thousands of significant entries, against the oracle.  Tokens, keep counts and
+id lists bit-exact; probabilities within 1e-6 relative (fp32 roundings of the
+same fp64 quotients)."""
+from __future__ import annotations
+
+import numpy as np
+import pytest
+
+from tensormark_amd import workloads
+from tests.helpers import params_array
+from tests.test_gpu_sample import check, run_gpu
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def ctx():
+    from tensormark_amd import Sampler
+
+    s = Sampler(max_batch=320, max_vocab=262144)
+    yield s
+    s.close()
+
+
+def _rows(rng, B, V, dtype, std, grid=0.0):
+    x = rng.normal(0.0, std, (B, V)).astype(np.float32)
+    x[np.arange(B)[:, None], rng.integers(0, V, (B, 6))] += rng.uniform(0, 12, (B, 6)).astype(np.float32)
+    if grid:
+        x = (np.round(x / grid) * grid).astype(np.float32)
+    if dtype == "bf16":
+        b = workloads.to_bf16_bits(x)
+        return b, workloads.bf16_bits_to_f32(b)
+    if dtype == "f16":
+        x = x.astype(np.float16)
+    return x, x.astype(np.float32)
+
+
+def _mixed(B, seed):
+    p = params_array(B, top_k=0, seed=np.arange(B) + seed)
+    p["temperature"] = np.resize([1.0, 0.7, 1.3, 1.0, 0.9, 1.0, 0.8, 1.0], B)
+    p["top_p"] = np.resize([1.0, 0.95, 0.999, 0.0, 1.0, 2.0, 0.5, 1.0], B)
+    p["min_p"] = np.resize([0.0, 0.0, 0.02, 0.0, 0.001, 0.0, 0.3, 0.0], B)
+    return p
+
+
+@pytest.mark.parametrize("dtype", ["f32", "f16", "bf16"])
+@pytest.mark.parametrize("V", [1300, 16384, 16385, 40963, 151936, 262144])
+def test_whole_vocabulary_rows(ctx, orc, dtype, V):
+    """Every way a row is decided (a cut, a min-p cut, top_p = 1's exact sums,
+    neither), with penalties, a mask and an id list, over one chunk to sixteen,
+    aligned and not."""
+    rng = np.random.default_rng(V)
+    B = 8
+    x, wide = _rows(rng, B, V, dtype, 1.5)
+    p = _mixed(B, V)
+    recent = mask = None
+    if V != 151936:   # (that one without a window: the packed stream)
+        p["repeat_penalty"], p["repeat_last_n"], p["frequency_penalty"] = 1.1, 100, 0.1
+        recent = rng.integers(0, V, (B, 120))
+        mask = workloads.mask_dense(rng, B, V, 0.8)
+    got = run_gpu(ctx, x, p, recent=recent, mask=mask, topk_cap=20, dtype=dtype)
+    want = orc.sample_batch(wide, p, recent=recent, mask=mask, topk_cap=20)
+    check(got, want, topk_cap=20)
+
+
+@pytest.mark.parametrize("grid", [0.125, 1.0, 64.0])
+def test_ties(ctx, orc, grid):
+    """Hundreds to all of a row's entries on one value: a cut or a draw inside
+    a run of equal logits, and rows whose buckets hold too many keys (the
+    full-row form)."""
+    B, V = 8, 50000
+    rng = np.random.default_rng(int(grid * 8))
+    x, wide = _rows(rng, B, V, "bf16", 1.5, grid)
+    p = _mixed(B, 5)
+    check(run_gpu(ctx, x, p, topk_cap=3, dtype="bf16"), orc.sample_batch(wide, p, topk_cap=3), topk_cap=3)
+
+
+def test_draws_at_the_ends(ctx, orc):
+    """Uniforms at 0, next to 1 and in between, so that the drawn entry is the
+    first, the last kept and far down the row."""
+    B, V = 12, 30011
+    rng = np.random.default_rng(3)
+    x, wide = _rows(rng, B, V, "f32", 2.0)
+    p = params_array(B, temperature=1.0, top_k=0, seed=1)
+    p["top_p"] = np.resize([1.0, 0.9], B)
+    hi = np.resize(np.repeat([0, 0xFFFFFFFF, 0xFFFFFF00, 0x80000000, 0xF0000000, 1], 2), B)
+    draws = np.stack([np.full(B, 0xFFFFFFFF), hi], axis=1).astype(np.uint32)
+    check(run_gpu(ctx, x, p, draws=draws), orc.sample_batch(wide, p, draws=draws))
+
+
+def test_more_rows_than_cus(ctx, orc):
+    """300 rows: no workgroups are left to help, each row's own takes every
+    range."""
+    B, V = 300, 6000
+    rng = np.random.default_rng(9)
+    x, wide = _rows(rng, B, V, "f16", 1.0)
+    p = _mixed(B, 11)
+    check(run_gpu(ctx, x, p, dtype="f16"), orc.sample_batch(wide, p))
+
+
+def test_calls_in_a_row_and_a_captured_graph(ctx):
+    """The row states and shared words of one call do not reach the next, and
+    a captured call replays to the eager result."""
+    import torch
+
+    B, V = 6, 70000
+    rng = np.random.default_rng(21)
+    x = torch.from_numpy(_rows(rng, B, V, "f32", 2.0)[0]).to("cuda:0")
+    p = ctx.params_tensor(_mixed(B, 2))
+    want = {k: v.clone() for k, v in ctx.sample(x, p).items()}
+    out = {k: torch.zeros_like(v) for k, v in want.items()}
+    s = torch.cuda.Stream()
+    with torch.cuda.stream(s):
+        ctx.sample(x, p, out=out)
+        g = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(g, stream=s):
+            ctx.sample(x, p, out=out)
+    torch.cuda.synchronize()
+    for _ in range(4):
+        for v in out.values():
+            v.zero_()
+        g.replay()
+        torch.cuda.synchronize()
+        assert all(torch.equal(out[k], want[k]) for k in want)
+        again = ctx.sample(x.flip(0).contiguous(), p)   # the program's own work between replays
+        torch.cuda.synchronize()
+        assert int(again["status"].abs().sum()) == 0
