@@ -15,8 +15,15 @@ namespace tms {
 constexpr int kSpecMaxK = 16;      // draft tokens per sequence
 constexpr int kSpecParts = 64;     // vocabulary parts of the residual draw
 constexpr int kPartWords = 3;      // u64 per part: weight sum, target sum, the bonus row's part max
+constexpr int kSpecPartIds = 32768;  // ids of a statistics part, where the rows fill the chip
+constexpr int kSpecFill = 1024;      // most statistics parts of a call with fewer rows than that
+constexpr int kSpecClaims = 8;       // claim counters of a verify launch
 constexpr int kCounterStride = 64; // u32 between per-row arrival counters: one 256-byte line
                                    // each, so the rows' atomics do not queue on one line
+// Words of spec_rparts: two for each part of each row of the largest call.
+constexpr size_t spec_rpart_words(size_t max_batch, int max_vocab) {
+    return 2 * (max_batch * (2 * kSpecMaxK + 1) * (((size_t)max_vocab + kSpecPartIds - 1) / kSpecPartIds) + kSpecFill);
+}
 }  // namespace tms
 
 // Statistics of one speculative-verify row (target or draft).
@@ -43,6 +50,8 @@ struct tms_context {
     uint32_t* spec_tickets;    // [max_batch][kCounterStride] verify arrival counters (word 0)
     uint64_t* spec_parts;      // [max_batch][kSpecParts][kPartWords] published partial sums
     tms_spec_stat* spec_stats; // [max_batch][2 * kSpecMaxK + 1]
+    uint64_t* spec_rparts;     // spec_rpart_words(): a row's part: its max word and its share of Z
+    uint32_t* spec_claims;     // [2][8][kCounterStride] claim counters of the row kernel and the resolve
     uint32_t* dlocks;          // [dense_slots] whole-row region locks
     int32_t* ov_n;             // [max_batch] history pre-pass: list lengths (-1: overflow)
     int32_t* ov_ids;           // [max_batch][TMS_HISTORY_MAX_IDS] listed ids

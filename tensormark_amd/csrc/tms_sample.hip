@@ -1313,7 +1313,9 @@ extern "C" int tms_create(int device, int max_batch, int max_vocab, tms_context*
     const size_t off_st = off_l + nc * tms::kListStride * sizeof(uint64_t);
     const size_t off_sp = off_st + nb * tms::kCounterStride * 4;   // one 256-byte line per ticket
     const size_t off_ss = off_sp + nb * tms::kSpecParts * tms::kPartWords * sizeof(uint64_t);
-    const size_t off_tl = off_ss + nb * (2 * tms::kSpecMaxK + 1) * sizeof(tms_spec_stat);
+    const size_t off_sr = off_ss + nb * (2 * tms::kSpecMaxK + 1) * sizeof(tms_spec_stat);
+    const size_t off_sc = off_sr + 256 * ((tms::spec_rpart_words(nb, max_vocab) * sizeof(uint64_t) + 255) / 256);
+    const size_t off_tl = off_sc + 2 * tms::kSpecClaims * tms::kCounterStride * sizeof(uint32_t);
     const size_t tl_chunks = (size_t)std::min(ctx->max_chunks, tms::kWideMaxChunksHost);
     const size_t off_dq = off_tl + nb * tl_chunks * tms::kWideListStride * sizeof(uint64_t);
     const size_t off_hn = off_dq + 256 * (((size_t)tms::kDenseSlotsMax * sizeof(uint32_t) + 255) / 256);
@@ -1354,6 +1356,8 @@ extern "C" int tms_create(int device, int max_batch, int max_vocab, tms_context*
     ctx->spec_tickets = (uint32_t*)(p + off_st);
     ctx->spec_parts = (uint64_t*)(p + off_sp);
     ctx->spec_stats = (tms_spec_stat*)(p + off_ss);
+    ctx->spec_rparts = (uint64_t*)(p + off_sr);
+    ctx->spec_claims = (uint32_t*)(p + off_sc);
     ctx->tlists = (uint64_t*)(p + off_tl);
     ctx->dlocks = (uint32_t*)(p + off_dq);
     ctx->ov_n = (int32_t*)(p + off_hn);

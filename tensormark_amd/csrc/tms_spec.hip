@@ -5,19 +5,20 @@
 //   statistics    one record per row (the k + 1 target rows and the k draft
 //                 rows of every sequence): m = max(v / T), the exact integer
 //                 sum Z of the row's weights q44(exp64(v / T - m)), and the
-//                 weight of the row's draft token.  16-byte aligned rows of
-//                 up to 64K fp32 (32K fp16/bf16) ids: spec_row_kernel, one
-//                 1024-thread workgroup per row holding the row in registers
-//                 (one read); other rows: spec_stats_kernel, two passes.
+//                 weight of the row's draft token.  spec_row_kernel: one
+//                 1024-thread workgroup per 32K ids of a row, holding them in
+//                 registers (one read), or per fewer ids where the rows are
+//                 too few to fill the chip.
 //   spec_resolve  B x P workgroups.  Every workgroup of a sequence evaluates
 //                 the accept tests u_i < p_t(x_i) / p_d(x_i) from the row
 //                 statistics (the same decision in each), then sums the
 //                 weights of its 1/P of the vocabulary for the distribution
 //                 the final draw uses: the residual max(p_t - p_d, 0) at the
 //                 first rejection, else the target row k (the bonus token).
-//                 It publishes the partial sums, takes a ticket, and the last
-//                 arriver finds the part holding the draw's threshold,
-//                 recomputes that part's weights and locates the token.
+//                 It publishes the partial sums, reads the others', and the
+//                 workgroup whose part holds the draw's threshold locates the
+//                 token (vocabularies past 262144: the last arriver by ticket
+//                 does, recomputing that part's weights).
 //
 // The weights are build-defined (no reference counterpart): exp64 is the
 // table-driven exponential of tms_device.h, q44 rounds to multiples of 2^-44,
@@ -29,6 +30,7 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <algorithm>
 #include <atomic>
 
 #include "../../include/tmsample_hip.h"
@@ -44,6 +46,13 @@ constexpr int kPartPoll = 1 << 20;            // bound on the finisher's wait pe
 constexpr int kRowT = 1024;          // threads of the row kernel
 constexpr int kRowW = kRowT / 64;
 
+// Workgroups that wait on each other, in a grid that need not be resident at
+// once, take their places in order from a counter: when one is resident, all
+// those before it have been, so the parts of every earlier row are all
+// running or done, and only the last row of a group's counter waits for
+// workgroups that have still to start, which those rows' ends let in.
+// kSpecClaims counters, each with the rows (or sequences) of its residue,
+// share the traffic.  The last claim resets its counter.
 struct SArgs {
     const void* target;
     const void* draft;
@@ -59,7 +68,11 @@ struct SArgs {
     int32_t* out_status;
     tms_spec_stat* stats;
     uint64_t* parts;
-    uint32_t* tickets;   // [B][kCounterStride]: resolve parts, or rows of the row kernel
+    uint32_t* tickets;   // [B][kCounterStride]: resolve parts
+    int S, pv;           // parts of a row in the row kernel, and their length in vectors
+    uint64_t* rparts;    // [B * (2k + 1)][S][2]: a part's max word and its share of Z
+    uint32_t* claims;    // [2][kSpecClaims][kCounterStride]: row kernel, resolve
+    bool claim_rows, claim_parts;   // the grid may not be resident at once
 #ifdef TMS_TRACE
     uint64_t* trace;     // trace builds: 8 stamps per workgroup
 #endif
@@ -85,7 +98,27 @@ struct SpecLds {
     tms_spec_stat srow[2 * kSpecMaxK + 1];
     int stok[kSpecMaxK];
     double su[kSpecMaxK];
+    int claim;
 };
+
+// This workgroup's place in a grid of kSpecClaims x n: (row, part) of rows
+// of S parts; claimed when the grid may not be resident at once.
+__device__ __forceinline__ void place(int S, bool claimed, uint32_t* counters, SpecLds& L, int& row, int& part) {
+    const int c = blockIdx.x & (kSpecClaims - 1);
+    int n = blockIdx.x / kSpecClaims;
+    if (claimed) {
+        if (threadIdx.x == 0) {
+            uint32_t* w = counters + c * kCounterStride;
+            const uint32_t m = __hip_atomic_fetch_add(w, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            if (m == gridDim.x / kSpecClaims - 1) st_agent(w, 0u);
+            L.claim = (int)m;
+        }
+        lds_sync();
+        n = L.claim;
+    }
+    row = n / S * kSpecClaims + c;
+    part = n % S;
+}
 
 __device__ __forceinline__ void load_exp_table(double* tab) {
     if (threadIdx.x < 64) tab[threadIdx.x] = kSpecExpTab[threadIdx.x];
@@ -152,8 +185,8 @@ __device__ __forceinline__ float block_max_f32(float v, float* sh) {
 
 template <int NW = kWaves>
 __device__ __forceinline__ int64_t block_sum_i64(int64_t v, int64_t* sh) {
-    v = wave_sum_i64(v);
-    if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = v;
+    v = wave_incl_scan_i64_dpp(v);
+    if ((threadIdx.x & 63) == 63) sh[threadIdx.x >> 6] = v;
     __syncthreads();
     int64_t r = 0;
 #pragma unroll
@@ -212,75 +245,42 @@ __device__ __forceinline__ int64_t as_i64(double f) {
     return __double_as_longlong(f + 0x1p52) - __double_as_longlong(0x1p52);
 }
 
-template <typename T>
-__global__ __launch_bounds__(kBlock) void spec_stats_kernel(SArgs a) {
-    __shared__ double tab[64];
-    __shared__ float shf[kWaves];
-    __shared__ int64_t shl[kWaves];
-    __shared__ int shi[kWaves];
-    load_exp_table(tab);
-    const int R = 2 * a.k + 1;
-    const int g = blockIdx.x;
-    const int b = g / R, i = g - b * R;
-    const T* row = spec_row<T>(a, b, i);
-    const float temp = a.params[b].temperature;
-
-    float mx = -__builtin_huge_valf();
-    int nf = 0;
-    for_range(row, 0, a.V, a.fast, [&](int, float v) {
-        nf |= __builtin_amdgcn_class(v, 0x203);   // NaN or +inf
-        mx = fmaxf(mx, scaled(v, temp));
-    });
-    mx = block_max_f32(mx, shf);   // also orders the table's LDS writes
-    nf = block_or(nf, shi);
-    int st = TMS_ROW_OK;
-    if (nf) st = TMS_ROW_NONFINITE;
-    else if (mx == -__builtin_huge_valf()) st = TMS_ROW_ALL_MASKED;
-    else if (mx == __builtin_huge_valf()) st = TMS_ROW_NONFINITE;
-    const double md = (double)mx;
-    int64_t z = 0;
-    if (st == TMS_ROW_OK) {
-        for_range(row, 0, a.V, a.fast, [&](int, float v) { z += weight(v, temp, md, tab); });
-        z = block_sum_i64(z, shl);
-    }
-    if (threadIdx.x == 0) {
-        const int di = i < a.k ? i : (i > a.k ? i - a.k - 1 : -1);
-        int64_t ex = 0;
-        if (st == TMS_ROW_OK && di >= 0) {
-            const int x = a.tokens[(int64_t)b * a.k + di];
-            if (x >= 0 && x < a.V) ex = weight(Elt<T>::scalar(row + x), temp, md, tab);
-        }
-        // Agent-scope stores, as the chunked statistics write theirs: rows on
-        // different XCDs share cache lines of the record array.
-        uint64_t* w = (uint64_t*)(a.stats + g);
-        st_agent(&w[0], (uint64_t)__float_as_uint(mx) | ((uint64_t)(uint32_t)st << 32));
-        st_agent(&w[1], (uint64_t)z);
-        st_agent(&w[2], (uint64_t)ex);
-        st_agent(&w[3], (uint64_t)0);
-    }
-}
-
 // Loops over a thread's registers (slot sl holds vector t + sl * NT, in
-// while below nv): the max of v / T and the NaN/+inf flag, then the share
-// of Z.
-template <typename T, int NS, int NT, bool DIV>
-__device__ __forceinline__ void row_max(const uint4 (&q)[NS], int nv, float temp, float& mx, int& nf) {
+// while below nv): the max of the logits and the NaN/+inf flag, then the
+// share of Z.
+//
+// Max and flag from the logits' bits, three integer operations a logit (two
+// of them to an instruction): a positive NaN is above +inf as a signed
+// number, a negative one above -inf as an unsigned one, and the maximum is
+// the signed maximum or, with every sign bit set, the unsigned minimum.  A
+// slot past nv holds a vector of the row again, which changes none of them.
+template <typename T, int NS>
+__device__ __forceinline__ void row_max(const uint4 (&q)[NS], float& mx, int& nf) {
     constexpr int VEC = Elt<T>::kVec;
-    const int t = threadIdx.x;
+    int hi = INT32_MIN;
+    uint32_t hu = 0, lu = UINT32_MAX;
 #pragma unroll
     for (int sl = 0; sl < NS; ++sl) {
-        const bool in = t + sl * NT < nv;
         float x[VEC];
         Elt<T>::widen(q[sl], x);
 #pragma unroll
         for (int e = 0; e < VEC; ++e) {
-            nf |= in ? __builtin_amdgcn_class(x[e], 0x203) : 0;   // NaN or +inf
-            mx = in ? fmaxf(mx, scaled<DIV>(x[e], temp)) : mx;
+            const uint32_t u = __float_as_uint(x[e]);
+            hi = max(hi, (int)u);
+            hu = max(hu, u);
+            lu = min(lu, u);
         }
     }
+    nf = hi >= 0x7F800000 || hu > 0xFF800000u;   // NaN or +inf
+    mx = __uint_as_float(hi >= 0 ? (uint32_t)hi : lu);
 }
+// DIV: v / T as (float)(v * y), y = RN(1 / T) in double.  The quotient of
+// two 24-bit significands is no midpoint of two floats and lies at least
+// 2^-49 of itself from one, and the product is within 2^-52 of it, so it
+// rounds to the float that the division returns.  (Subnormal quotients can
+// be midpoints: there the two may differ by 2^-149, which moves no weight.)
 template <typename T, int NS, int NT, bool DIV>
-__device__ __forceinline__ int64_t row_z(const uint4 (&q)[NS], int nv, float temp, double md, const double* tab) {
+__device__ __forceinline__ int64_t row_z(const uint4 (&q)[NS], int nv, double y, double md, const double* tab) {
     constexpr int VEC = Elt<T>::kVec;
     const int t = threadIdx.x;
     // whole numbers of at most 2^44 each, at most 128 of them: the double
@@ -293,10 +293,49 @@ __device__ __forceinline__ int64_t row_z(const uint4 (&q)[NS], int nv, float tem
         Elt<T>::widen(q[sl], x);
         if (t + sl * NT < nv) {
 #pragma unroll
-            for (int e = 0; e < VEC; ++e) z += q44_exp_nonpos_f((double)scaled<DIV>(x[e], temp) - md, tab);
+            for (int e = 0; e < VEC; ++e) {
+                const double v = (double)x[e];
+                z += q44_exp_nonpos_f((DIV ? (double)(float)(v * y) : v) - md, tab);
+            }
         }
     }
     return __double_as_longlong(z + 0x1p52) - __double_as_longlong(0x1p52);
+}
+
+// 16 bytes of logits at any element's address.
+template <typename T>
+__device__ __forceinline__ uint4 ld_vec(const T* p) {
+    struct __attribute__((packed, aligned(sizeof(T)))) Q { uint32_t x, y, z, w; };
+    const Q q = *(const Q*)p;
+    return make_uint4(q.x, q.y, q.z, q.w);
+}
+
+// The vector with its first n elements (n < the vector width) set to -inf.
+template <typename T>
+__device__ __forceinline__ uint4 drop_first(uint4 q, int n) {
+    constexpr uint32_t kNeg = Elt<T>::kNegInfWord;
+    constexpr int PW = 4 / (int)sizeof(T);   // elements a word
+    uint32_t w[4] = {q.x, q.y, q.z, q.w};
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        if (n >= (i + 1) * PW) w[i] = kNeg;
+        else if (PW == 2 && n == 2 * i + 1) w[i] = (w[i] & 0xFFFF0000u) | (kNeg & 0xFFFFu);
+    }
+    return make_uint4(w[0], w[1], w[2], w[3]);
+}
+
+// A row of fewer ids than a vector holds: its logits, then -inf.
+template <typename T>
+__device__ __forceinline__ uint4 short_row(const T* row, int V) {
+    uint4 q;
+    T* e = (T*)&q;
+    uint32_t* w = (uint32_t*)&q;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) w[i] = Elt<T>::kNegInfWord;
+#pragma unroll
+    for (int i = 0; i < Elt<T>::kVec; ++i)
+        if (i < V) e[i] = row[i];
+    return q;
 }
 
 // The sequence's statistics, draft tokens and accept uniforms staged in LDS
@@ -315,9 +354,16 @@ __device__ void accept_tests(const SArgs& a, int b, SpecLds& L, int& status, int
         const uint64_t w0 = ld_agent(&w[0]);
         L.srow[t].m = __uint_as_float((uint32_t)w0);
         L.srow[t].status = (int32_t)(w0 >> 32);
-        L.srow[t].Z = (int64_t)ld_agent(&w[1]);
+        L.srow[t].Z = a.S > 1 ? 0 : (int64_t)ld_agent(&w[1]);
         L.srow[t].ex = (int64_t)ld_agent(&w[2]);
         L.srow[t].pad = 0;
+    }
+    if (a.S > 1) {   // the shares of Z of a row's parts
+        __syncthreads();
+        const uint64_t* w = a.rparts + (int64_t)g0 * a.S * 2;
+        for (int i = t; i < R * a.S; i += kBlock)
+            if (!(a.lazy && i / a.S == a.k))
+                atomicAdd((unsigned long long*)&L.srow[i / a.S].Z, (unsigned long long)ld_agent(&w[2 * i + 1]));
     }
     if (t < a.k) {
         L.stok[t] = a.tokens[(int64_t)b * a.k + t];
@@ -375,7 +421,7 @@ __device__ void accept_tests(const SArgs& a, int b, SpecLds& L, int& status, int
 }
 
 // Part p of sequence b's resolution.
-// WAIT (the whole grid resident at once, runs of at most kRunMax ids): every
+// WAIT (up to kSpecParts parts of runs of at most kRunMax ids): every
 // workgroup keeps its part's weights in registers, reads every part's sums
 // (bounded wait), and the one whose part holds the draw's threshold locates
 // the token from its registers; the last reader (by a done counter) zeroes
@@ -395,6 +441,11 @@ __device__ void resolve_part(const SArgs& a, int b, int p, SpecLds& L) {
     const uint32_t* dw = a.draws ? a.draws + (int64_t)b * (a.k + 1) * 2 : nullptr;
     int status, acc, rej;
     SPEC_TR(0);
+    // the rows' part maxima, ready for the next call (their readers, the
+    // statistics' workgroups, have ended)
+    if (a.S > 1 && p == 0)
+        for (int i = t; i < (2 * a.k + 1) * a.S; i += kBlock)
+            st_agent(a.rparts + ((int64_t)b * (2 * a.k + 1) * a.S + i) * 2, (uint64_t)0);
     accept_tests<T>(a, b, L, status, acc, rej);
     SPEC_TR(1);
     if (status != TMS_ROW_OK) {
@@ -421,14 +472,35 @@ __device__ void resolve_part(const SArgs& a, int b, int p, SpecLds& L) {
     int64_t wr[kRunMax], er[kRunMax];   // WAIT: the run's draw and target weights
     if constexpr (WAIT) {
         // a contiguous run of ids per thread, every load issued at once
-        const int E = (hi - lo + kBlock - 1) / kBlock;
+        const int E = a.Lp / kBlock;   // a multiple of the vector width
         const int r_lo = min(hi, lo + t * E), r_hi = min(hi, r_lo + E);
         float xt[kRunMax], xd[kRunMax];
 #pragma unroll
-        for (int j = 0; j < kRunMax; ++j) {
-            const int id = min(r_lo + j, hi - 1);
-            xt[j] = j < E ? Elt<T>::scalar(rt + id) : 0.0f;
-            xd[j] = (j < E && rej >= 0) ? Elt<T>::scalar(rd + id) : 0.0f;
+        for (int j = 0; j < kRunMax; ++j) xt[j] = xd[j] = 0.0f;
+        if (r_hi - r_lo == E) {
+            constexpr int VEC = Elt<T>::kVec;
+#pragma unroll
+            for (int j = 0; j < kRunMax; j += VEC) {
+                if (j >= E) break;
+                const uint4 qt = ld_vec(rt + r_lo + j);
+                uint4 qd = qt;
+                if (rej >= 0) qd = ld_vec(rd + r_lo + j);
+                float x[VEC];
+                Elt<T>::widen(qt, x);
+#pragma unroll
+                for (int e = 0; e < VEC; ++e) xt[j + e] = x[e];
+                Elt<T>::widen(qd, x);
+#pragma unroll
+                for (int e = 0; e < VEC; ++e) xd[j + e] = x[e];
+            }
+        } else {   // the row's last run
+#pragma unroll
+            for (int j = 0; j < kRunMax; ++j) {
+                if (r_lo + j < r_hi) {
+                    xt[j] = Elt<T>::scalar(rt + r_lo + j);
+                    if (rej >= 0) xd[j] = Elt<T>::scalar(rd + r_lo + j);
+                }
+            }
         }
         double mtu = mt;
         if (a.lazy && rej < 0) {
@@ -623,7 +695,7 @@ __device__ void resolve_part(const SArgs& a, int b, int p, SpecLds& L) {
     SPEC_TR(6);
     // The part's weights, a contiguous run of ids per thread.
     const int plo = ps * a.Lp, phi = min(a.V, plo + a.Lp);
-    const int E = (phi - plo + kBlock - 1) / kBlock;
+    const int E = WAIT ? a.Lp / kBlock : (phi - plo + kBlock - 1) / kBlock;
     const int my_lo = min(phi, plo + t * E), my_hi = min(phi, my_lo + E);
     auto w_at = [&](int id) -> int64_t {
         const double et = weight_f(Elt<T>::scalar(rt + id), temp, mt, tab);
@@ -711,51 +783,85 @@ template <typename T, bool WAIT>
 __global__ __launch_bounds__(kBlock) void spec_resolve_kernel(SArgs a) {
     __shared__ SpecLds L;
     load_exp_table(L.tab);
-    resolve_part<T, WAIT>(a, blockIdx.x / a.P, blockIdx.x % a.P, L);
+    int b, p;
+    place(a.P, WAIT && a.claim_parts, a.claims + kSpecClaims * kCounterStride, L, b, p);
+    if (b < a.B) resolve_part<T, WAIT>(a, b, p, L);
 }
 
-// Row statistics for 16-byte aligned rows of at most kRowT x NS vectors:
-// one 1024-thread workgroup per row holds the row in registers (one read)
-// and writes the row's record: m = max(v / T), the status,
-// Z = sum of q44(exp64(v / T - m)) and the draft token's weight, equal to
-// spec_stats_kernel's.  Two workgroups per CU (64 registers a thread) up to
-// 8 vectors a thread.  The parts-wise resolve follows on the stream.
-template <typename T, int NS>
-__global__ __launch_bounds__(kRowT) __attribute__((amdgpu_waves_per_eu(NS <= 8 ? 8 : 4, 8)))
+// Row statistics: S workgroups a row (a.S), each holding its part of the row
+// in registers (one read), in at most NS vectors a thread.  With more than
+// one part, each publishes its maximum and waits for the others' (place()
+// has the order that lets it).  Part 0 writes the row's record: m = max(v /
+// T) = max(v) / T (a correctly rounded division by T > 0 is monotone), the
+// status and the draft token's weight; every part adds its share of
+// Z = sum of q44(exp64(v / T - m)), whole numbers, so any split sums to the
+// same.  64 registers a thread: 32 waves a CU.
+//
+// Bound by the exponentials: 110 cycles of a SIMD for 64 of them, 34 us of
+// the 63 that B = 32, k = 5, V = 151936 bf16 takes (as two passes by one
+// 256-thread workgroup a row: 125); the rest is the loads and the exchange
+// that a part's exponentials wait for, under the other workgroup's of its CU.
+// Parts of 16K ids in 512-thread workgroups measured alike (88 us a call
+// against 92, but 42 against 41 at B = 32, k = 8, V = 32000 fp32).  B = 1, k
+// = 4, V = 128256 bf16: 9 rows in 16 parts each take 8.3 us (59).
+template <typename T, int NS, int NT>
+__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(8, 8)))
 void spec_row_kernel(SArgs a) {
     constexpr int VEC = Elt<T>::kVec;
+    constexpr int NW = NT / 64;
     __shared__ SpecLds L;
     load_exp_table(L.tab);
     const int t = threadIdx.x;
     // lazy: 2k rows a sequence (the bonus row k left to the resolve)
     const int R = a.lazy ? 2 * a.k : 2 * a.k + 1;
-    const int g = blockIdx.x;
+    int g = blockIdx.x, p = 0;
+    if (a.S > 1) {
+        place(a.S, a.claim_rows, a.claims, L, g, p);
+        if (g >= a.B * R) return;
+    }
     const int b = g / R;
     int i = g - b * R;
     if (a.lazy && i >= a.k) ++i;
     const T* row = spec_row<T>(a, b, i);
-    const float temp = a.params[b].temperature;
-    const bool div = temp != 1.0f;
-    const int nv = a.V / VEC;
+    const int V = a.V;
+    const int v0 = p * a.pv;
+    const int nv = min((V + VEC - 1) / VEC - v0, a.pv);   // this part's vectors
     uint4 q[NS];
+    if (V >= VEC) {
+        // a ragged row's last vector ends at the row's end
 #pragma unroll
-    for (int sl = 0; sl < NS; ++sl) q[sl] = *(const uint4*)(row + (int64_t)min(t + sl * kRowT, nv - 1) * VEC);
+        for (int sl = 0; sl < NS; ++sl)
+            q[sl] = ld_vec(row + min((v0 + min(t + sl * NT, nv - 1)) * VEC, V - VEC));
+        if (!a.fast) {   // ... and begins with ids of the vector before it
+#pragma unroll
+            for (int sl = 0; sl < NS; ++sl) {
+                const int dup = (v0 + t + sl * NT) * VEC - (V - VEC);
+                if (dup > 0 && dup < VEC) q[sl] = drop_first<T>(q[sl], dup);
+            }
+        }
+    } else {
+#pragma unroll
+        for (int sl = 0; sl < NS; ++sl) q[sl] = short_row(row, V);
+    }
     // The draft token's logit (draft rows; target row i takes draft i's
     // token), loaded now, after the stream's loads: it is in flight under
     // the max and the sums, and its weight is formed at the end.
     const int di = i < a.k ? i : (i > a.k ? i - a.k - 1 : -1);
     bool xin = false;
     float xv = 0.0f;
-    if (t == 0 && di >= 0) {
+    if (t == 0 && p == 0 && di >= 0) {
         const int x = a.tokens[(int64_t)b * a.k + di];
-        xin = x >= 0 && x < a.V;
+        xin = x >= 0 && x < V;
         if (xin) xv = Elt<T>::scalar(row + x);
     }
-    float mx = -__builtin_huge_valf();
-    int nf = 0;
-    if (div) row_max<T, NS, kRowT, true>(q, nv, temp, mx, nf);
-    else row_max<T, NS, kRowT, false>(q, nv, temp, mx, nf);
-    // The row's maximum and NaN/+inf flag in one exchange: each wave's pair
+    float mx;
+    int nf;
+    row_max<T, NS>(q, mx, nf);
+    if constexpr (VEC == 8) {   // not the max's widened logits, which take twice the registers, kept for the sums
+#pragma unroll
+        for (int sl = 0; sl < NS; ++sl) asm("" : "+v"(q[sl].x), "+v"(q[sl].y), "+v"(q[sl].z), "+v"(q[sl].w));
+    }
+    // The part's maximum and NaN/+inf flag in one exchange: each wave's pair
     // in LDS words written once, so one barrier (which also orders the
     // table's LDS writes) and none after the reads.
     {
@@ -769,29 +875,65 @@ void spec_row_kernel(SArgs a) {
         mx = L.shf[0];
         nf = L.misc[0];
 #pragma unroll
-        for (int i = 1; i < kRowW; ++i) {
-            mx = fmaxf(mx, L.shf[i]);
-            nf |= L.misc[i];
+        for (int j = 1; j < NW; ++j) {
+            mx = fmaxf(mx, L.shf[j]);
+            nf |= L.misc[j];
         }
     }
+    int bad = 0;
+    uint64_t* rp = a.rparts + ((int64_t)b * (2 * a.k + 1) + i) * a.S * 2;
+    if (a.S > 1) {   // the row's, from every part's word
+        if (t == 0) st_agent(rp + 2 * p, kPartReady | ((uint64_t)nf << 32) | okey(mx));
+        if (t < 64) {
+            uint32_t km = 0;
+            for (int j = t; j < a.S; j += 64) {
+                uint64_t h = 0;
+                for (int it = 0; it < kPartPoll; ++it) {
+                    h = ld_agent(rp + 2 * j);
+                    if (h & kPartReady) break;
+                    __builtin_amdgcn_s_sleep(1);
+                }
+                bad |= (h & kPartReady) ? 0 : 1;
+                nf |= (int)((h >> 32) & 1u);
+                km = max(km, (uint32_t)h);
+            }
+            km = (uint32_t)wave_max_u64(km);
+            nf = __any(nf) ? 1 : 0;
+            bad = __any(bad) ? 1 : 0;
+            if (t == 0) {
+                L.stok[0] = (int)km;
+                L.stok[1] = nf | bad << 1;
+            }
+        }
+        lds_sync();
+        mx = okey_inv((uint32_t)L.stok[0]);
+        nf = L.stok[1] & 1;
+        bad = L.stok[1] >> 1;
+    }
+    const float temp = a.params[b].temperature;
+    const bool div = temp != 1.0f;
+    mx = scaled(mx, temp);
     int st = TMS_ROW_OK;
-    if (nf) st = TMS_ROW_NONFINITE;
+    if (bad) st = TMS_ROW_INTERNAL;
+    else if (nf) st = TMS_ROW_NONFINITE;
     else if (mx == -__builtin_huge_valf()) st = TMS_ROW_ALL_MASKED;
     else if (mx == __builtin_huge_valf()) st = TMS_ROW_NONFINITE;
     const double md = (double)mx;
     int64_t z = 0;
     if (st == TMS_ROW_OK)
-        z = div ? row_z<T, NS, kRowT, true>(q, nv, temp, md, L.tab) : row_z<T, NS, kRowT, false>(q, nv, temp, md, L.tab);
+        z = div ? row_z<T, NS, NT, true>(q, nv, 1.0 / (double)temp, md, L.tab)
+                : row_z<T, NS, NT, false>(q, nv, 1.0, md, L.tab);
     {   // Z: each wave's share in LDS words written once (one barrier)
-        const int64_t wz = wave_sum_i64(z);
-        if ((t & 63) == 0) L.shl[t >> 6] = wz;
+        const int64_t wz = wave_incl_scan_i64_dpp(z);
+        if ((t & 63) == 63) L.shl[t >> 6] = wz;
         lds_sync();
         z = 0;
         if (t == 0)
 #pragma unroll
-            for (int i = 0; i < kRowW; ++i) z += L.shl[i];
+            for (int j = 0; j < NW; ++j) z += L.shl[j];
     }
-    if (t == 0) {
+    if (t == 0 && a.S > 1) st_agent(rp + 2 * p + 1, (uint64_t)z);
+    if (t == 0 && p == 0) {
         const int64_t ex = (st == TMS_ROW_OK && xin) ? weight(xv, temp, md, L.tab) : 0;
         uint64_t* w = (uint64_t*)(a.stats + (int64_t)b * (2 * a.k + 1) + i);
         st_agent(&w[0], (uint64_t)__float_as_uint(mx) | ((uint64_t)(uint32_t)st << 32));
@@ -803,26 +945,81 @@ void spec_row_kernel(SArgs a) {
 
 }  // namespace tms
 
-// Whether a resolve grid of n workgroups is resident at once on the current
-// device (occupancy of the waiting form x compute units, looked up once per
-// device and type): the waiting form's workgroups wait on each other.
-template <typename T>
-static bool resolve_resident(int n) {
+// Workgroups of a kernel that are resident at once on the current device
+// (occupancy x compute units, looked up once per device and kernel); 0 if
+// it cannot be told.
+template <auto Kernel, int NT>
+static int resident_cap() {
     constexpr int kMaxDevices = 64;
     static std::atomic<int> cap[kMaxDevices];
     int dev = 0;
-    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kMaxDevices) return false;
+    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kMaxDevices) return 0;
     int c = cap[dev].load(std::memory_order_relaxed);
     if (c == 0) {
         int per_cu = 0, cus = 0;
-        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, tms::spec_resolve_kernel<T, true>, tms::kBlock, 0) !=
-                hipSuccess ||
+        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, Kernel, NT, 0) != hipSuccess ||
             hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
-            return false;
-        c = per_cu * cus > 0 ? per_cu * cus : -1;
+            return 0;
+        c = per_cu * cus;
         cap[dev].store(c, std::memory_order_relaxed);
     }
-    return c > 0 && n <= c;
+    return c;
+}
+
+template <typename T>
+static int launch_verify(tms::SArgs s, hipStream_t stream) {
+    constexpr int VEC = tms::Elt<T>::kVec;
+    constexpr int NSMAX = tms::kSpecPartIds / VEC / tms::kRowT;
+    const int R = 2 * s.k + 1;
+    const int nv = (s.V + VEC - 1) / VEC;
+    // The resolve: the waiting form for up to kSpecParts parts of kRunMax ids
+    // a thread, in parts of half that length where its grid is resident at
+    // once (B = 1, V = 128256: 10 us).  B = 32, V = 151936 bf16: 27 us, where
+    // the ticket form, which reads the threshold's part again, takes 35.
+    const int cap2 = resident_cap<tms::spec_resolve_kernel<T, true>, tms::kBlock>();
+    const int most = tms::kBlock * tms::kRunMax;
+    s.Lp = most / 2;
+    s.P = (s.V + s.Lp - 1) / s.Lp;
+    if (s.P > tms::kSpecParts || s.B * s.P > cap2) {
+        s.Lp = most;
+        s.P = (s.V + s.Lp - 1) / s.Lp;
+    }
+    const bool wait = s.P <= tms::kSpecParts && s.P <= cap2 / tms::kSpecClaims;
+    if (!wait) {
+        s.P = std::min((s.V + 2047) / 2048, tms::kSpecParts);
+        s.Lp = ((s.V + s.P - 1) / s.P + 7) / 8 * 8;
+        s.P = (s.V + s.Lp - 1) / s.Lp;
+    }
+    s.claim_parts = wait && s.B * s.P > cap2;
+    const int n2 = (s.B + tms::kSpecClaims - 1) / tms::kSpecClaims * tms::kSpecClaims * s.P;
+    // The statistics: as few parts a row as registers allow, more where the
+    // rows would leave compute units idle.  Where the grid takes more than
+    // one round of the chip, the waiting resolve takes the bonus rows'
+    // statistics itself: 2k rows a sequence in place of 2k + 1, for an
+    // exchange more (B = 32, k = 8, V = 32000 fp32: 512 rows, one round of
+    // two workgroups a CU, in place of 544).
+    const int cap1 = resident_cap<tms::spec_row_kernel<T, NSMAX, tms::kRowT>, tms::kRowT>();
+    s.S = (nv + NSMAX * tms::kRowT - 1) / (NSMAX * tms::kRowT);
+    const int fill = std::min(cap1 / 2, tms::kSpecFill) / (s.B * R);
+    s.S = std::max(s.S, std::min(fill, (nv + tms::kRowT - 1) / tms::kRowT));
+    s.pv = (nv + s.S - 1) / s.S;
+    s.S = (nv + s.pv - 1) / s.pv;
+    s.lazy = wait && s.B * R * s.S > cap1;
+    const int rows = s.B * (s.lazy ? R - 1 : R);
+    const int n1 = s.S == 1 ? rows : (rows + tms::kSpecClaims - 1) / tms::kSpecClaims * tms::kSpecClaims * s.S;
+    s.claim_rows = n1 > cap1;
+    const dim3 g1((unsigned)n1), b1(tms::kRowT), g2((unsigned)n2), b2(tms::kBlock);
+    if (s.pv <= tms::kRowT)
+        hipLaunchKernelGGL((tms::spec_row_kernel<T, 1, tms::kRowT>), g1, b1, 0, stream, s);
+    else if (s.pv <= NSMAX / 2 * tms::kRowT)
+        hipLaunchKernelGGL((tms::spec_row_kernel<T, NSMAX / 2, tms::kRowT>), g1, b1, 0, stream, s);
+    else
+        hipLaunchKernelGGL((tms::spec_row_kernel<T, NSMAX, tms::kRowT>), g1, b1, 0, stream, s);
+    if (wait)
+        hipLaunchKernelGGL((tms::spec_resolve_kernel<T, true>), g2, b2, 0, stream, s);
+    else
+        hipLaunchKernelGGL((tms::spec_resolve_kernel<T, false>), g2, b2, 0, stream, s);
+    return hipGetLastError() == hipSuccess ? TMS_OK : TMS_ERR_HIP;
 }
 
 extern "C" int tms_spec_verify(tms_context* ctx, const tms_spec_args* a, hipStream_t stream) {
@@ -848,11 +1045,6 @@ extern "C" int tms_spec_verify(tms_context* ctx, const tms_spec_args* a, hipStre
     s.V = a->vocab;
     s.fast = ((uintptr_t)a->target_logits % 16 == 0) && ((uintptr_t)a->draft_logits % 16 == 0) &&
              (a->vocab % vec == 0);
-    // Parts of about 2K ids, at most kSpecParts, each a multiple of 8 ids.
-    int P = (a->vocab + 2047) / 2048;
-    P = P < 1 ? 1 : (P > tms::kSpecParts ? tms::kSpecParts : P);
-    s.Lp = ((a->vocab + P - 1) / P + 7) / 8 * 8;
-    s.P = (a->vocab + s.Lp - 1) / s.Lp;
     s.tokens = a->draft_tokens;
     s.params = a->params;
     s.draws = a->draws;
@@ -865,46 +1057,11 @@ extern "C" int tms_spec_verify(tms_context* ctx, const tms_spec_args* a, hipStre
 #ifdef TMS_TRACE
     s.trace = tms::g_spec_trace;
 #endif
-    // 16-byte aligned rows of at most kRowT x 16 vectors (fp32) or x 4
-    // (fp16, bf16: 8 spill): the row kernel (two workgroups per CU up to 8
-    // vectors a thread); others: the per-row statistics.  Then the resolve.
-    const int R = 2 * a->k + 1;
-    const int slots = (a->vocab / vec + tms::kRowT - 1) / tms::kRowT;
-    const int max_ns = esz == 4 ? 16 : 4;
-    const int row_ns = (!s.fast || slots > max_ns) ? 0 : slots <= 4 ? 4 : slots <= 8 ? 8 : 16;
-    const dim3 block(tms::kBlock);
-    const dim3 g2((unsigned)(a->batch * s.P));
-    const dim3 brow(tms::kRowT);
-    // The waiting resolve (its grid resident at once, runs of at most
-    // kRunMax ids) takes the bonus rows' statistics itself when the row
-    // kernel runs: 2k rows a sequence there (config 4: 512 rows, one round
-    // of two workgroups per CU, in place of 544).
-#define TMS_SPEC_LAUNCH(T, NS2, NS3)                                                       \
-    do {                                                                                   \
-        const bool wait = resolve_resident<T>(a->batch * s.P) &&                          \
-                          (s.Lp + tms::kBlock - 1) / tms::kBlock <= tms::kRunMax;          \
-        s.lazy = wait && row_ns > 0;                                                       \
-        const dim3 g1((unsigned)(a->batch * (s.lazy ? R - 1 : R)));                        \
-        if (row_ns > 0) {                                                                  \
-            if (row_ns == 4)                                                               \
-                hipLaunchKernelGGL((tms::spec_row_kernel<T, 4>), g1, brow, 0, stream, s);  \
-            else if (row_ns == 8)                                                          \
-                hipLaunchKernelGGL((tms::spec_row_kernel<T, NS2>), g1, brow, 0, stream, s);\
-            else                                                                           \
-                hipLaunchKernelGGL((tms::spec_row_kernel<T, NS3>), g1, brow, 0, stream, s);\
-        } else {                                                                           \
-            hipLaunchKernelGGL(tms::spec_stats_kernel<T>, g1, block, 0, stream, s);        \
-        }                                                                                  \
-        if (wait)                                                                          \
-            hipLaunchKernelGGL((tms::spec_resolve_kernel<T, true>), g2, block, 0, stream, s);  \
-        else                                                                               \
-            hipLaunchKernelGGL((tms::spec_resolve_kernel<T, false>), g2, block, 0, stream, s); \
-    } while (0)
+    s.rparts = ctx->spec_rparts;
+    s.claims = ctx->spec_claims;
     switch (a->dtype) {
-        case TMS_DTYPE_F32: TMS_SPEC_LAUNCH(float, 8, 16); break;
-        case TMS_DTYPE_F16: TMS_SPEC_LAUNCH(_Float16, 4, 4); break;   // row_ns is 4 or 0
-        default: TMS_SPEC_LAUNCH(tms::Bf16, 4, 4); break;              // row_ns is 4 or 0
+        case TMS_DTYPE_F32: return launch_verify<float>(s, stream);
+        case TMS_DTYPE_F16: return launch_verify<_Float16>(s, stream);
+        default: return launch_verify<tms::Bf16>(s, stream);
     }
-#undef TMS_SPEC_LAUNCH
-    return hipGetLastError() == hipSuccess ? TMS_OK : TMS_ERR_HIP;
 }

@@ -213,3 +213,34 @@ def test_spec_bonus_row_statistics_in_the_resolve(orc, sampler):
     check_spec(orc, gpu, target, draft, tokens, params, words)
     assert gpu["status"][0] == 2 and gpu["status"][2] == 3
     assert (gpu["status"][3:] == 0).all() and (gpu["accepted"][3:] == k).all()
+
+
+@pytest.mark.parametrize("dtype,B,V,k", [
+    ("bf16", 1, 151937, 4), ("f16", 2, 70003, 1), ("f32", 3, 32769, 2),   # parts that fill idle units
+    ("f32", 2, 3, 2), ("bf16", 2, 7, 1), ("f16", 3, 9, 3),                # around one 16-byte vector
+    ("bf16", 96, 66001, 2),                                               # places claimed in both launches
+    ("f32", 72, 33001, 2),                                                # two parts a row, resident resolve
+    ("f16", 2, 262145, 1),                                                # the ticket form of the resolve
+])
+def test_spec_rows_in_parts(orc, sampler, dtype, B, V, k):
+    """Rows whose statistics several workgroups share, odd vocabularies (rows
+    at any element's address, a ragged last vector), and grids that are not
+    resident at once: twice, since the second call takes the words that the
+    first left."""
+    if V > 262144:
+        from tensormark_amd import Sampler
+
+        sampler = Sampler(max_batch=B, max_vocab=V)
+    rng = np.random.default_rng(V + B)
+    target = rng.standard_normal((B, k + 1, V), dtype=np.float32) * 2.0
+    draft = target[:, :k] + 0.7 * rng.standard_normal((B, k, V), dtype=np.float32)
+    tokens = workloads.softmax_draws(rng, draft)
+    params = params_array(B, temperature=1.0, seed=np.arange(B) + 11)
+    params["temperature"] = rng.choice([0.7, 1.0, 1.3], size=B)
+    if B > 1:
+        target[B - 1, 0, V - 1] = np.nan      # the last part of a row
+        draft[0, k - 1, : V - 1] = -np.inf    # one id left, in the last vector
+    words = philox_words(orc, params, k)
+    for _ in range(2):
+        gpu = run_spec(sampler, target, draft, tokens, params, dtype=dtype)
+        check_spec(orc, gpu, target, draft, tokens, params, words, dtype)
