@@ -43,7 +43,8 @@
 
 namespace tms {
 
-constexpr int kHBlock = 256;
+constexpr int kHBlock = 1024;
+constexpr int kHStage = 4096;             // most recent ids of the history held in LDS
 constexpr int kHSlots = 2 * kHistMax;
 constexpr uint32_t kHCount = 0xFFFFu;     // window count
 constexpr uint32_t kHDry = 1u << 30;      // a DRY target
@@ -72,18 +73,17 @@ struct HistArgs {
 };
 
 struct HistLds {
-    uint32_t key[kHSlots];     // id + 1; 0 = empty (before the table: DRY's staged window)
+    uint32_t key[kHSlots];     // id + 1; 0 = empty (before the table: DRY's window past kHStage)
     uint32_t info[kHSlots];    // kHCount | kHDry | kHBan
-    uint16_t ent[kHSlots];     // the slot's entry
     uint16_t eslot[kHistMax];  // the entry's slot
     float val[kHistMax];
+    int32_t win[kHStage];      // the last ids of the history, newest first
     int32_t tslot[kHBlock];    // DRY: one tile of target slots, in position order
-    int32_t tk[kHBlock];       //      and their exponents L - allowed_length
+    float tsub[kHBlock];       //      and what each takes off: multiplier * base^(L - allowed_length)
     uint16_t dlen[kDryMax];    // DRY: the match length at each window position
-    uint32_t dbrk[kDryMax / 32];   // DRY: staged window positions holding a breaker
+    uint32_t dbrk[kDryMax / 32 + 1];   // DRY: staged window positions holding a breaker
     int wave_i[kHBlock / 64];
     int flag;                  // overflow
-    int found;
 };
 
 __device__ __forceinline__ uint32_t hslot0(int id) {
@@ -114,8 +114,9 @@ __device__ __forceinline__ int hfind(const HistLds& L, int id) {
     return -1;
 }
 
+// The OR of every thread's two low bits.
 __device__ __forceinline__ int block_or(int v, HistLds& L) {
-    v = __any(v) ? 1 : 0;
+    v = (__any(v & 1) ? 1 : 0) | (__any(v & 2) ? 2 : 0);
     if ((threadIdx.x & 63) == 0) L.wave_i[threadIdx.x >> 6] = v;
     __syncthreads();
     int r = 0;
@@ -149,32 +150,41 @@ __device__ __forceinline__ bool is_breaker(const uint8_t* brk, int V, int id) {
 
 // DRY match lengths (tmsample.h:159-163) of every window position i <
 // last = dn - 1: how far the runs ending at i and at last agree, never
-// across a breaker.  r[j] is the window's id at last - j (staged in the
-// table's key array), bit j of dbrk marks a breaker there; the length at i
-// is the common prefix of r and r[last - i ..], which stops at the window's
-// start (position d + k <= last).  Lengths go to L.dlen[i].
+// across a breaker.  r[j] is the window's id at last - j, bit j of dbrk
+// marks a breaker there; the length at i is the common prefix of r and
+// r[last - i ..], which stops at the window's start (position d + k <=
+// last).  Lengths go to L.dlen[i].
 __device__ __forceinline__ bool dry_eq(const int32_t* r, const uint32_t* brk, int a, int b) {
     return r[a] == r[b] && !((brk[a >> 5] >> (a & 31)) & 1u) && !((brk[b >> 5] >> (b & 31)) & 1u);
 }
 
-__device__ void dry_lengths(const int32_t* dw, int dn, const uint8_t* breaker, int V, HistLds& L) {
+// The breaker bits of positions j .. j + 7, from bit 0.
+__device__ __forceinline__ uint32_t brk_bits(const uint32_t* brk, int j) {
+    return (uint32_t)((((uint64_t)brk[(j >> 5) + 1] << 32) | brk[j >> 5]) >> (j & 31));
+}
+
+__device__ void dry_lengths(const int32_t* r, int dn, HistLds& L) {
     const int t = threadIdx.x, lane = t & 63;
     const int last = dn - 1;
-    int32_t* r = (int32_t*)L.key;
-    for (int i = t; i < kDryMax / 32; i += kHBlock) L.dbrk[i] = 0u;
-    __syncthreads();
-    for (int j = t; j < dn; j += kHBlock) {
-        const int id = dw[last - j];
-        r[j] = id;
-        if (is_breaker(breaker, V, id)) atomicOr(&L.dbrk[j >> 5], 1u << (j & 31));
-    }
-    __syncthreads();
     int over = 0;
     for (int i = t; i < last; i += kHBlock) {
         const int d = last - i;
         int k = 0;
-        while (k < kDryDirect && d + k < dn && dry_eq(r, L.dbrk, k, d + k)) ++k;
-        over |= k == kDryDirect ? 1 : 0;
+        // the first id, then eight at a time, their loads together
+        if (dry_eq(r, L.dbrk, 0, d)) {
+            for (;;) {
+                uint32_t ne = brk_bits(L.dbrk, k) | brk_bits(L.dbrk, d + k);
+#pragma unroll
+                for (int j = 0; j < 8; ++j) {
+                    const int b = d + k + j;
+                    ne |= (b >= dn || r[k + j] != r[min(b, last)] ? 1u : 0u) << j;
+                }
+                ne &= 0xFFu;
+                k += ne ? __builtin_ctz(ne) : 8;
+                if (ne || k >= kDryDirect) break;
+            }
+        }
+        over |= k >= kDryDirect ? 1 : 0;
         L.dlen[i] = (uint16_t)k;
     }
     if (!block_or(over, L)) return;
@@ -205,6 +215,13 @@ __device__ void dry_lengths(const int32_t* dw, int dn, const uint8_t* breaker, i
     __syncthreads();
 }
 
+// One row's steps are a chain of short passes over the window, the list and
+// the table, bound by the latency of each: 1024 threads take a window of
+// that many ids in one go, the ids and their breaker bits are read from
+// memory once, and DRY's terms are formed where their positions are listed,
+// so that an entry's subtractions wait on no load.  B = 16, 1024 ids, V =
+// 128256 bf16, n-gram ban and DRY: 17 us (256 threads, each pass reading
+// the history again and an entry its exponents' scales one by one: 35).
 template <typename T>
 __global__ __launch_bounds__(kHBlock) void history_kernel(HistArgs a) {
     __shared__ HistLds L;
@@ -224,28 +241,55 @@ __global__ __launch_bounds__(kHBlock) void history_kernel(HistArgs a) {
                         nrec >= H.dry_allowed_length + 1 &&
                         min(nrec, H.dry_penalty_last_n) >= H.dry_allowed_length + 1;
     const int dn = dry_on ? min(nrec, H.dry_penalty_last_n) : 0;
-    const int32_t* dw = rec + (nrec - dn);
     const int dlast = dn - 1;
     // every exponent L - allowed_length is below dn - allowed_length
     if (dry_on && (dn > kDryMax || (a.dry_scale && a.dry_scale_stride < dn - H.dry_allowed_length))) {
         if (t == 0) a.ov_n[row] = -1;   // the row reports TMS_ROW_UNSUPPORTED
         return;
     }
-    if (dry_on) dry_lengths(dw, dn, a.breaker, V, L);
-
-    {
+    // The newest ids, newest first, and the breakers' bits of DRY's window.
+    // A window of more goes over the table's keys, which are cleared after.
+    const int ns = min(nrec, kHStage);
+    const bool big = dn > kHStage;
+    int32_t* r = big ? (int32_t*)L.key : L.win;
+    if (dry_on) {
+        for (int i = t; i <= kDryMax / 32; i += kHBlock) L.dbrk[i] = 0u;
+        lds_sync();
+    }
+    for (int j = t; j < max(ns, dn); j += kHBlock) {
+        const int id = rec[nrec - 1 - j];
+        if (j < ns) L.win[j] = id;
+        if (big && j < dn) r[j] = id;
+        if (j < dn && is_breaker(a.breaker, V, id)) atomicOr(&L.dbrk[j >> 5], 1u << (j & 31));
+    }
+    if (t == 0) {
+        L.flag = 0;
+    }
+    auto clear = [&] {
         uint4* k4 = (uint4*)L.key;
         uint4* i4 = (uint4*)L.info;
         for (int i = t; i < kHSlots / 4; i += kHBlock) {
             k4[i] = make_uint4(0, 0, 0, 0);
             i4[i] = make_uint4(0, 0, 0, 0);
         }
-        if (t == 0) {
-            L.flag = 0;
-            L.found = 0;
-        }
+    };
+    if (!big) clear();
+    lds_sync();
+    if (dry_on) dry_lengths(r, dn, L);
+    if (big) {
+        lds_sync();
+        clear();
+        lds_sync();
     }
-    __syncthreads();
+    // the history's id at position p, and what DRY takes off at window
+    // position i: the id after it, -1 for none
+    auto rec_at = [&](int p) { return nrec - 1 - p < ns ? L.win[nrec - 1 - p] : rec[p]; };
+    auto dry_id = [&](int i) {
+        const int j = dlast - 1 - i;
+        if (L.dlen[i] < H.dry_allowed_length || ((L.dbrk[j >> 5] >> (j & 31)) & 1u)) return -1;
+        const int id = rec_at(nrec - 1 - j);
+        return id < V ? id : -1;
+    };
     int full = 0;
 
     // ---- repetition / frequency / presence window: counts per id
@@ -259,7 +303,7 @@ __global__ __launch_bounds__(kHBlock) void history_kernel(HistArgs a) {
     if (pn.on) {
         const int from = nrec > P.repeat_last_n ? nrec - P.repeat_last_n : 0;
         for (int p = from + t; p < nrec; p += kHBlock) {
-            const int id = rec[p];
+            const int id = rec_at(p);
             if (id < 0 || id >= V) continue;
             const int s = hinsert(L, id);
             if (s < 0) full = 1;
@@ -274,9 +318,9 @@ __global__ __launch_bounds__(kHBlock) void history_kernel(HistArgs a) {
         const int m = ng - 1, s0 = nrec - m;
         for (int i = t; i < s0; i += kHBlock) {
             bool same = true;
-            for (int k = 0; k < m && same; ++k) same = rec[i + k] == rec[s0 + k];
+            for (int k = 0; k < m && same; ++k) same = rec_at(i + k) == rec_at(s0 + k);
             if (!same) continue;
-            const int id = rec[i + m];
+            const int id = rec_at(i + m);
             if (id < 0 || id >= V) continue;
             const int s = hinsert(L, id);
             if (s < 0) full = 1;
@@ -287,9 +331,8 @@ __global__ __launch_bounds__(kHBlock) void history_kernel(HistArgs a) {
     // ---- DRY targets (tmsample.h:150-169)
     if (dry_on) {
         for (int i = t; i < dlast; i += kHBlock) {
-            if (L.dlen[i] < H.dry_allowed_length) continue;
-            const int id = dw[i + 1];
-            if (id < 0 || id >= V || is_breaker(a.breaker, V, id)) continue;
+            const int id = dry_id(i);
+            if (id < 0) continue;
             const int s = hinsert(L, id);
             if (s < 0) full = 1;
             else atomicOr(&L.info[s], kHDry);
@@ -299,20 +342,29 @@ __global__ __launch_bounds__(kHBlock) void history_kernel(HistArgs a) {
     __syncthreads();
 
     // ---- number the slots (the list, in slot order)
-    constexpr int kPer = kHSlots / kHBlock;   // 32 consecutive slots per thread
+    constexpr int kPer = kHSlots / kHBlock;   // consecutive slots per thread
+    uint32_t key[kPer];
     int mine = 0;
-#pragma unroll 8
-    for (int j = 0; j < kPer; ++j) mine += L.key[t * kPer + j] != 0u ? 1 : 0;
+#pragma unroll
+    for (int j = 0; j < kPer; j += 4) {
+        const uint4 q = *(const uint4*)&L.key[t * kPer + j];
+        key[j] = q.x;
+        key[j + 1] = q.y;
+        key[j + 2] = q.z;
+        key[j + 3] = q.w;
+    }
+#pragma unroll
+    for (int j = 0; j < kPer; ++j) mine += key[j] != 0u ? 1 : 0;
     int n = 0;
     int e = hist_excl_scan(mine, n, L);
     if (L.flag || n > kHistMax) {
         if (t == 0) a.ov_n[row] = -1;   // the row reports TMS_ROW_UNSUPPORTED
         return;
     }
+#pragma unroll
     for (int j = 0; j < kPer; ++j) {
         const int s = t * kPer + j;
-        if (L.key[s] != 0u) {
-            L.ent[s] = (uint16_t)e;
+        if (key[j] != 0u) {
             L.eslot[e] = (uint16_t)s;
             ++e;
         }
@@ -329,15 +381,15 @@ __global__ __launch_bounds__(kHBlock) void history_kernel(HistArgs a) {
         const bool allowed = (mrow[id >> 5] >> (id & 31)) & 1u;
         float v = allowed ? Elt<T>::scalar(base + id) : NEG_INF;
         const uint32_t c = f & kHCount;
-        if (allowed && c) v = apply_pen(v, c, pn);
+        if (allowed && c) v = apply_pen<true>(v, c, pn);
         L.val[i] = v;
         if (f & kHBan) banned = 1;
         else if (v > NEG_INF) alive = 1;
     }
-    banned = block_or(banned, L);
+    const int any = block_or(banned | alive << 1, L);
+    alive = any >> 1;
     bool restore = false;
-    if (banned) {
-        alive = block_or(alive, L);
+    if (any & 1) {
         if (!alive) {
             // an allowed id outside the list with a logit above -inf?
             const int words = (V + 31) >> 5;
@@ -375,22 +427,21 @@ __global__ __launch_bounds__(kHBlock) void history_kernel(HistArgs a) {
         const float* scale = a.dry_scale ? a.dry_scale + (int64_t)row * a.dry_scale_stride : nullptr;
         for (int i0 = 0; i0 < dlast; i0 += kHBlock) {
             const int i = i0 + t;
-            int slot = -1, k = 0;
+            int slot = -1;
+            float sub = 0.0f;
             if (i < dlast) {
-                const int Lr = L.dlen[i];
-                if (Lr >= H.dry_allowed_length) {
-                    const int id = dw[i + 1];
-                    if (id >= 0 && id < V && !is_breaker(a.breaker, V, id)) {
-                        slot = hfind(L, id);
-                        k = Lr - H.dry_allowed_length;
-                    }
+                const int id = dry_id(i);
+                if (id >= 0) {
+                    const int k = L.dlen[i] - H.dry_allowed_length;
+                    sub = mult * (scale ? scale[k] : tms_dry_scale(dbase, k));
+                    slot = hfind(L, id);
                 }
             }
             int nh = 0;
             const int pos = hist_excl_scan(slot >= 0 ? 1 : 0, nh, L);
             if (slot >= 0) {
                 L.tslot[pos] = slot;
-                L.tk[pos] = k;
+                L.tsub[pos] = sub;
             }
             __syncthreads();
             if (nh) {
@@ -398,9 +449,9 @@ __global__ __launch_bounds__(kHBlock) void history_kernel(HistArgs a) {
                     const int s = L.eslot[q];
                     if (!(L.info[s] & kHDry)) continue;
                     float v = L.val[q];
+#pragma unroll 4
                     for (int j = 0; j < nh; ++j)
-                        if (L.tslot[j] == s)
-                            v -= mult * (scale ? scale[L.tk[j]] : tms_dry_scale(dbase, L.tk[j]));
+                        if (L.tslot[j] == s) v -= L.tsub[j];
                     L.val[q] = v;
                 }
             }

@@ -113,12 +113,43 @@ struct Pen {
     const float* ov = nullptr;
 };
 
+// v divided by rep `cnt` times (v <= 0: multiplied), each result rounded: a
+// chain of as many divisions as the id occurs, 100 and more for a text's
+// commonest words.  A quotient in the normal range comes from a product with
+// y = RN(1 / rep) in double: v / rep is no midpoint of two floats (a
+// midpoint's odd 25-bit significand does not divide v's) and so lies at
+// least 2^-49 of itself from one, and the product is within 2^-52 of it.
+// Below the normal range, the division itself.  Four steps to a branch: one
+// to a branch loses half of what the products give.
+__device__ __forceinline__ float divide_times(float v, float rep, uint32_t cnt) {
+    if (cnt >= 8) {   // (fewer divisions cost less than the reciprocal)
+        const double y = 1.0 / (double)rep;
+        for (; cnt >= 4; cnt -= 4) {
+            float q = v;
+#pragma unroll
+            for (int j = 0; j < 4; ++j) q = (float)((double)q * y);
+            if (q < FLT_MIN) break;   // (the quotients fall: the last is the least)
+            v = q;
+        }
+        if (!(v > 0.f))
+            for (; cnt > 0; --cnt) v *= rep;
+    }
+    for (; cnt > 0; --cnt) v = v > 0.f ? v / rep : v * rep;
+    return v;
+}
+
 // Repetition penalty applied `cnt` times (tmsample.h:61), then frequency and
 // presence: v -= (float)cnt * freq + presence.  With pn.ov, the pre-pass's
-// value of list entry cnt - 1.
+// value of list entry cnt - 1.  LONG: by divide_times, in the history
+// pre-pass (250 listed ids of a 1024-id history: 11 us by divisions, 4) and
+// the wide top-k kernel (B = 64, V = 128256 with 256-id windows: 15.0 us a
+// call by divisions, 13.9); the sparse-mask kernel, whose windows hold few of the
+// allowed ids, measured 0.3 us slower with it, from the code's size alone.
+template <bool LONG = false>
 __device__ __forceinline__ float apply_pen(float v, uint32_t cnt, const Pen& pn) {
     if (pn.ov) return pn.ov[cnt - 1];
-    if (pn.rep_on)
+    if (pn.rep_on && LONG) v = divide_times(v, pn.rep, cnt);
+    else if (pn.rep_on)
         for (uint32_t r = 0; r < cnt; ++r) v = v > 0.f ? v / pn.rep : v * pn.rep;
     if (pn.fp_on) {
         const float t1 = (float)cnt * pn.freq;

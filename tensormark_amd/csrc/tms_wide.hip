@@ -583,7 +583,7 @@ __attribute__((amdgpu_waves_per_eu(kSlots == 4 ? 8 : NT / 256, 8))) void topk_wi
     // entries already meet
     float own_v = NEG_INF;
     if (owner) {
-        own_v = apply_pen(own_x, sm.wtab[wslot] & ((1u << kCntBits) - 1u), pn);
+        own_v = apply_pen<true>(own_x, sm.wtab[wslot] & ((1u << kCntBits) - 1u), pn);
         if (!(own_v < __builtin_huge_valf()) && own_v != NEG_INF) atomicOr(&sm.onf, 1);
     }
     WTR(3);

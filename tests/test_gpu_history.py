@@ -337,3 +337,50 @@ def test_dry_long_repetitive_windows(sampler, orc):
     assert dt < 1.0, dt
     assert g["status"][3] == 4 and g["tokens"][3] == -1
     check(g, want, 8, rows=[0, 1, 2])
+
+
+@pytest.mark.parametrize("n,last_n", [(1, 1), (3, 3), (1023, 1023), (1025, 1025), (4096, 4096),
+                                      (4097, 4096), (4097, 4097), (6001, 300), (8200, 8192)])
+def test_history_window_edges(sampler, orc, n, last_n):
+    """Histories and DRY windows around one pass of the workgroup and around
+    the ids it holds in LDS: older ids are read where they are needed, and a
+    DRY window of more of them is staged elsewhere."""
+    rng = np.random.default_rng(n + last_n)
+    B, V = 4, 50000
+    recent = _repeating(rng, B, n, 12, flip=0.2)
+    recent[:, rng.integers(0, n)] = [-1, V, 3, 4]
+    x = rng.normal(0.0, 2.0, (B, V)).astype(np.float32)
+    _boost(x, recent, V)
+    breaker = np.zeros(V, np.uint8)
+    breaker[recent[2, 0]] = 1
+    p = params_array(B, temperature=0.9, top_k=40, top_p=0.95, seed=np.arange(B) + 17)
+    p["repeat_penalty"] = 1.1
+    p["repeat_last_n"] = [n, 5000, 64, 4097]
+    h = make_history(B, no_repeat_ngram=3, dry_multiplier=0.3, dry_base=1.01,
+                     dry_penalty_last_n=last_n)
+    want = orc.sample_batch(x, p, recent=recent, history=h, dry_breaker=breaker, topk_cap=8)
+    g = _run(sampler, x, p, recent=recent, history=h, breaker=breaker, topk_cap=8)
+    check(g, want, 8)
+
+
+@pytest.mark.parametrize("n", [7, 8, 11, 12, 300, 1500])
+@pytest.mark.parametrize("pre_pass", [False, True])
+def test_long_repetition_chains(sampler, orc, n, pre_pass):
+    """An id that occurs n times is divided n times, each quotient rounded:
+    around the count from which products stand in for the divisions, and
+    through the end of the normal range (2.0 / 1.1^1500 is subnormal), with
+    and without the history pre-pass."""
+    rng = np.random.default_rng(n)
+    B, V = 6, 20000
+    x = rng.normal(0.0, 1.0, (B, V)).astype(np.float32)
+    x[:, 5] = [1e30, 7.3, 2.0, -0.7, 1e-37, 0.0]
+    x[:, 6] = [8.0, 1.9, 0.3, 0.2, 2.0, 2.0]
+    recent = np.full((B, n + 3), 5, np.int32)
+    recent[:, ::7] = rng.integers(0, V, recent[:, ::7].shape)
+    p = params_array(B, temperature=0.8, top_k=20, top_p=0.95, seed=np.arange(B) + 5)
+    p["repeat_penalty"] = [1.3, 1.01, 1.1, 1.001, 1.1, 2.0]
+    p["repeat_last_n"] = n + 3
+    h = make_history(B, no_repeat_ngram=4) if pre_pass else None
+    want = orc.sample_batch(x, p, recent=recent, history=h, topk_cap=20)
+    g = _run(sampler, x, p, recent=recent, history=h, topk_cap=20)
+    check(g, want, 20)
