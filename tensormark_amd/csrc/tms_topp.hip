@@ -272,7 +272,8 @@ __device__ __forceinline__ int fetch(const KArgs& a, const Row& R, int3 j0, int3
 // registers, 16 a thread: the window's ids leave the stream and come back
 // penalised (apply_pen) from the first position to count them, then one pass
 // adds every entry's mass and count to its bucket (LDS atomics, four
-// exponentials in flight) and one places its id.
+// exponentials in flight; the count before is its place there) and one
+// writes its id.
 template <typename T>
 __device__ __forceinline__ void record(const KArgs& a, const Row& R, const tms_row_params& P, int c, Lds& L) {
     constexpr int VEC = Elt<T>::kVec, NV = kHistIds / kT, NVT = NV / VEC;
@@ -324,7 +325,7 @@ __device__ __forceinline__ void record(const KArgs& a, const Row& R, const tms_r
             if (w & 0x8000u) continue;   // another position of the id has it
             if (!((mrow[(e0 + o) >> 5] >> ((e0 + o) & 31)) & 1u)) continue;
             // (with the history pre-pass: the value of list position p)
-            const float v = apply_pen(Elt<T>::scalar(base + o), ovm ? (uint32_t)(p + 1) : w, pn);
+            const float v = apply_pen<true>(Elt<T>::scalar(base + o), ovm ? (uint32_t)(p + 1) : w, pn);
             const int x = atomicAdd(&L.misc[0], 1);
             if (x < kHistExtra) H.ext[x] = (uint64_t)__float_as_uint(v) << 32 | (uint32_t)(e0 + o);
         }
@@ -385,11 +386,16 @@ __device__ __forceinline__ void record(const KArgs& a, const Row& R, const tms_r
         lg = R.divide ? v / R.temp : v;
         return v == NEG ? kHistBuckets - 1 : min(top - topp_bucket(lg), kHistBuckets - 1);
     };
-    auto add = [&](int jb, double w) {
+    // jb: the bucket, with the entry's place in it (the count before) above
+    static_assert(kHistBuckets == 1024 && kHistIds + kHistExtra < 1 << 21, "bucket and place in 31 bits");
+    auto add = [&](int& jb, double w) {
         if (jb < kHistBuckets - 1) {
             __hip_atomic_fetch_add(&H.mass[jb], w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-            __hip_atomic_fetch_add(&H.cnt[jb], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+            jb |= (int)atomicAdd(&H.cnt[jb], 1u) << 10;
         }
+    };
+    auto place = [&](int jb, int local) {
+        if (jb != kHistBuckets - 1) H.ids[H.cnt[jb & (kHistBuckets - 1)] + (jb >> 10)] = (uint16_t)local;
     };
     int jb[NV];
 #pragma unroll
@@ -410,11 +416,17 @@ __device__ __forceinline__ void record(const KArgs& a, const Row& R, const tms_r
         for (int u = 0; u < 4; ++u) add(jb[g + u], w[u]);
         __builtin_amdgcn_sched_barrier(0);
     }
-    for (int i = t; i < tail + nx; i += kT) {
-        int local;
-        float lg;
-        const int b = bucket(odd(i, local), lg);
-        add(b, exp_span(fmax((double)lg - (double)lmax, -42.0), L.tab));
+    static_assert(VEC + kHistExtra <= 2 * kT, "two odd entries a thread");
+    int jo[2], lo[2];
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+        const int i = t + u * kT;
+        jo[u] = kHistBuckets - 1;
+        if (i < tail + nx) {
+            float lg;
+            jo[u] = bucket(odd(i, lo[u]), lg);
+            add(jo[u], exp_span(fmax((double)lg - (double)lmax, -42.0), L.tab));
+        }
     }
     lds_sync();
     int total;
@@ -426,15 +438,9 @@ __device__ __forceinline__ void record(const KArgs& a, const Row& R, const tms_r
     for (int i = t; i < nx; i += kT) st_agent(&rec[kHistExt + i], H.ext[i]);
     lds_sync();
 #pragma unroll
-    for (int g = 0; g < NV; ++g)
-        if (jb[g] < kHistBuckets - 1)
-            H.ids[atomicAdd(&H.cnt[jb[g]], 1u)] = (uint16_t)((t + g / VEC * kT) * VEC + g % VEC);
-    for (int i = t; i < tail + nx; i += kT) {
-        int local;
-        float lg;
-        const int b = bucket(odd(i, local), lg);
-        if (b < kHistBuckets - 1) H.ids[atomicAdd(&H.cnt[b], 1u)] = (uint16_t)local;
-    }
+    for (int g = 0; g < NV; ++g) place(jb[g], (t + g / VEC * kT) * VEC + g % VEC);
+#pragma unroll
+    for (int u = 0; u < 2; ++u) place(jo[u], lo[u]);
     lds_sync();
     for (int i = t; i < (total + 3) / 4; i += kT) st_agent(&rec[kHistId + i], ((const uint64_t*)H.ids)[i]);
     if (t == 0) st_agent(&rec[kHistHead], (uint64_t)(lost ? 0 : 1) << 32 | __float_as_uint(lmax));
