@@ -490,6 +490,14 @@ struct Elt<Bf16> {
     __device__ static float scalar(const Bf16* p) { return __uint_as_float((uint32_t)p->bits << 16); }
 };
 
+// 16 bytes of logits at any element's address.
+template <typename T>
+__device__ __forceinline__ uint4 ld_any(const T* p) {
+    struct __attribute__((packed, aligned(sizeof(T)))) Q { uint32_t x, y, z, w; };
+    const Q q = *(const Q*)p;
+    return make_uint4(q.x, q.y, q.z, q.w);
+}
+
 // Relaxed agent-scope accesses: coherent across the XCDs' L2 caches.
 template <typename U>
 __device__ __forceinline__ void st_agent(U* p, U v) {

@@ -1623,7 +1623,7 @@ constexpr size_t kNaHistIds = kNaHistN + align32(kNoAllocRows / 2);
 constexpr size_t kNaHistVals = kNaHistIds + (size_t)kNoAllocRows * tms::kHistMax / 2;
 constexpr size_t kNaOnes = kNaHistVals + (size_t)kNoAllocRows * tms::kHistMax / 2;
 constexpr size_t kNaDense = kNaOnes + align32(kNoAllocVocab / 64);
-constexpr size_t kNaWords = kNaDense + 2 * (size_t)kNoAllocVocab;   // 21.0 MB
+constexpr size_t kNaWords = kNaDense + 2 * (size_t)kNoAllocVocab;   // 11.7 MB
 }  // namespace
 
 static __device__ __align__(256) uint64_t scratch[kNaWords];

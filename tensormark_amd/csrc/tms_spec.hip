@@ -302,14 +302,6 @@ __device__ __forceinline__ int64_t row_z(const uint4 (&q)[NS], int nv, double y,
     return __double_as_longlong(z + 0x1p52) - __double_as_longlong(0x1p52);
 }
 
-// 16 bytes of logits at any element's address.
-template <typename T>
-__device__ __forceinline__ uint4 ld_vec(const T* p) {
-    struct __attribute__((packed, aligned(sizeof(T)))) Q { uint32_t x, y, z, w; };
-    const Q q = *(const Q*)p;
-    return make_uint4(q.x, q.y, q.z, q.w);
-}
-
 // The vector with its first n elements (n < the vector width) set to -inf.
 template <typename T>
 __device__ __forceinline__ uint4 drop_first(uint4 q, int n) {
@@ -482,9 +474,9 @@ __device__ void resolve_part(const SArgs& a, int b, int p, SpecLds& L) {
 #pragma unroll
             for (int j = 0; j < kRunMax; j += VEC) {
                 if (j >= E) break;
-                const uint4 qt = ld_vec(rt + r_lo + j);
+                const uint4 qt = ld_any(rt + r_lo + j);
                 uint4 qd = qt;
-                if (rej >= 0) qd = ld_vec(rd + r_lo + j);
+                if (rej >= 0) qd = ld_any(rd + r_lo + j);
                 float x[VEC];
                 Elt<T>::widen(qt, x);
 #pragma unroll
@@ -831,7 +823,7 @@ void spec_row_kernel(SArgs a) {
         // a ragged row's last vector ends at the row's end
 #pragma unroll
         for (int sl = 0; sl < NS; ++sl)
-            q[sl] = ld_vec(row + min((v0 + min(t + sl * NT, nv - 1)) * VEC, V - VEC));
+            q[sl] = ld_any(row + min((v0 + min(t + sl * NT, nv - 1)) * VEC, V - VEC));
         if (!a.fast) {   // ... and begins with ids of the vector before it
 #pragma unroll
             for (int sl = 0; sl < NS; ++sl) {

@@ -200,14 +200,6 @@ __device__ __forceinline__ int block_min(int v, Lds& L) {   // v >= 0
     return uni(r);
 }
 
-// 16 bytes at any element's address (rows of an odd vocabulary start anywhere).
-template <typename T>
-__device__ __forceinline__ uint4 ld_any(const T* p) {
-    struct __attribute__((packed, aligned(sizeof(T)))) Q { uint32_t x, y, z, w; };
-    const Q q = *(const Q*)p;
-    return make_uint4(q.x, q.y, q.z, q.w);
-}
-
 // put(i, v, id) for the entries i in [0, m) of the buckets [j0, j1] of nI
 // intervals, interval by interval: each chunk holds an interval's ids as
 // one run, so a thread's entries are found by index, U in flight.  Returns

@@ -384,3 +384,31 @@ def test_long_repetition_chains(sampler, orc, n, pre_pass):
     want = orc.sample_batch(x, p, recent=recent, history=h, topk_cap=20)
     g = _run(sampler, x, p, recent=recent, history=h, topk_cap=20)
     check(g, want, 20)
+
+
+@pytest.mark.parametrize("dtype", ["f32", "f16", "bf16"])
+@pytest.mark.parametrize("V", [3, 7, 8, 9, 4099, 16385, 32771, 65549])
+def test_ragged_rows_with_windows(sampler, orc, dtype, V):
+    """Rows at any element's address and a last vector of 1 to 7 ids, whose
+    maximum is the row's last id: top-k rows with a window and a mask."""
+    rng = np.random.default_rng(V)
+    B = 3
+    x = rng.normal(0.0, 2.0, (B, V)).astype(np.float32)
+    x[:, V - 1] = [20.0, 12.0, 9.0]
+    x[:, V - 2] = [3.0, 12.0, 9.5]
+    if dtype == "bf16":
+        gx = workloads.to_bf16_bits(x)
+        x = workloads.bf16_bits_to_f32(gx)
+    else:
+        gx = x
+        x = x.astype(np.float16).astype(np.float32) if dtype == "f16" else x
+    recent = rng.integers(0, V, (B, 64)).astype(np.int32)
+    recent[1] = V - 1
+    mask = np.full((B, (V + 31) // 32), 0xFFFFFFFF, np.uint32)
+    mask[2, (V - 1) >> 5] &= ~np.uint32(1 << ((V - 1) & 31))
+    p = params_array(B, temperature=0.9, top_k=20, top_p=0.95, seed=np.arange(B) + 7)
+    p["repeat_penalty"] = 1.1
+    p["greedy"] = [1, 0, 0]
+    want = orc.sample_batch(x, p, recent=recent, mask=mask, topk_cap=8)
+    g = _run(sampler, gx, p, recent=recent, mask=mask, topk_cap=8, dtype=dtype)
+    check(g, want, 8)
