@@ -11,19 +11,12 @@
 #include <stddef.h>
 #include <stdint.h>
 
+#include "tms_spec_plan.h"
+
 namespace tms {
-constexpr int kSpecMaxK = 16;      // draft tokens per sequence
-constexpr int kSpecParts = 64;     // vocabulary parts of the residual draw
 constexpr int kPartWords = 3;      // u64 per part: weight sum, target sum, the bonus row's part max
-constexpr int kSpecPartIds = 32768;  // ids of a statistics part, where the rows fill the chip
-constexpr int kSpecFill = 1024;      // most statistics parts of a call with fewer rows than that
-constexpr int kSpecClaims = 8;       // claim counters of a verify launch
 constexpr int kCounterStride = 64; // u32 between per-row arrival counters: one 256-byte line
                                    // each, so the rows' atomics do not queue on one line
-// Words of spec_rparts: two for each part of each row of the largest call.
-constexpr size_t spec_rpart_words(size_t max_batch, int max_vocab) {
-    return 2 * (max_batch * (2 * kSpecMaxK + 1) * (((size_t)max_vocab + kSpecPartIds - 1) / kSpecPartIds) + kSpecFill);
-}
 }  // namespace tms
 
 // Statistics of one speculative-verify row (target or draft).

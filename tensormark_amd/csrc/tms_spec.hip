@@ -30,7 +30,6 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
-#include <algorithm>
 #include <atomic>
 
 #include "../../include/tmsample_hip.h"
@@ -43,7 +42,6 @@ __constant__ double kSpecExpTab[64] = {TMS_EXP2_64THS};
 constexpr uint64_t kPartReady = 1ull << 63;   // published partial sum is complete
 constexpr int kPartPoll = 1 << 20;            // bound on the finisher's wait per part
 
-constexpr int kRowT = 1024;          // threads of the row kernel
 constexpr int kRowW = kRowT / 64;
 
 // Workgroups that wait on each other, in a grid that need not be resident at
@@ -419,7 +417,6 @@ __device__ void accept_tests(const SArgs& a, int b, SpecLds& L, int& status, int
 // the token from its registers; the last reader (by a done counter) zeroes
 // the parts.  Otherwise the last arriver by ticket gathers the parts and
 // recomputes the weights of the part holding the threshold.
-constexpr int kRunMax = 16;
 template <typename T, bool WAIT>
 __device__ void resolve_part(const SArgs& a, int b, int p, SpecLds& L) {
     const double* tab = L.tab;
@@ -962,52 +959,25 @@ template <typename T>
 static int launch_verify(tms::SArgs s, hipStream_t stream) {
     constexpr int VEC = tms::Elt<T>::kVec;
     constexpr int NSMAX = tms::kSpecPartIds / VEC / tms::kRowT;
-    const int R = 2 * s.k + 1;
-    const int nv = (s.V + VEC - 1) / VEC;
-    // The resolve: the waiting form for up to kSpecParts parts of kRunMax ids
-    // a thread, in parts of half that length where its grid is resident at
-    // once (B = 1, V = 128256: 10 us).  B = 32, V = 151936 bf16: 27 us, where
-    // the ticket form, which reads the threshold's part again, takes 35.
-    const int cap2 = resident_cap<tms::spec_resolve_kernel<T, true>, tms::kBlock>();
-    const int most = tms::kBlock * tms::kRunMax;
-    s.Lp = most / 2;
-    s.P = (s.V + s.Lp - 1) / s.Lp;
-    if (s.P > tms::kSpecParts || s.B * s.P > cap2) {
-        s.Lp = most;
-        s.P = (s.V + s.Lp - 1) / s.Lp;
-    }
-    const bool wait = s.P <= tms::kSpecParts && s.P <= cap2 / tms::kSpecClaims;
-    if (!wait) {
-        s.P = std::min((s.V + 2047) / 2048, tms::kSpecParts);
-        s.Lp = ((s.V + s.P - 1) / s.P + 7) / 8 * 8;
-        s.P = (s.V + s.Lp - 1) / s.Lp;
-    }
-    s.claim_parts = wait && s.B * s.P > cap2;
-    const int n2 = (s.B + tms::kSpecClaims - 1) / tms::kSpecClaims * tms::kSpecClaims * s.P;
-    // The statistics: as few parts a row as registers allow, more where the
-    // rows would leave compute units idle.  Where the grid takes more than
-    // one round of the chip, the waiting resolve takes the bonus rows'
-    // statistics itself: 2k rows a sequence in place of 2k + 1, for an
-    // exchange more (B = 32, k = 8, V = 32000 fp32: 512 rows, one round of
-    // two workgroups a CU, in place of 544).
-    const int cap1 = resident_cap<tms::spec_row_kernel<T, NSMAX, tms::kRowT>, tms::kRowT>();
-    s.S = (nv + NSMAX * tms::kRowT - 1) / (NSMAX * tms::kRowT);
-    const int fill = std::min(cap1 / 2, tms::kSpecFill) / (s.B * R);
-    s.S = std::max(s.S, std::min(fill, (nv + tms::kRowT - 1) / tms::kRowT));
-    s.pv = (nv + s.S - 1) / s.S;
-    s.S = (nv + s.pv - 1) / s.pv;
-    s.lazy = wait && s.B * R * s.S > cap1;
-    const int rows = s.B * (s.lazy ? R - 1 : R);
-    const int n1 = s.S == 1 ? rows : (rows + tms::kSpecClaims - 1) / tms::kSpecClaims * tms::kSpecClaims * s.S;
-    s.claim_rows = n1 > cap1;
-    const dim3 g1((unsigned)n1), b1(tms::kRowT), g2((unsigned)n2), b2(tms::kBlock);
-    if (s.pv <= tms::kRowT)
+    static_assert(tms::kSpecBlock == tms::kBlock, "the plan's resolve block");
+    const tms::SpecPlan p = tms::spec_plan(
+        s.B, s.k, s.V, VEC, resident_cap<tms::spec_row_kernel<T, NSMAX, tms::kRowT>, tms::kRowT>(),
+        resident_cap<tms::spec_resolve_kernel<T, true>, tms::kBlock>());
+    s.P = p.P;
+    s.Lp = p.Lp;
+    s.claim_parts = p.claim_parts;
+    s.S = p.S;
+    s.pv = p.pv;
+    s.lazy = p.lazy;
+    s.claim_rows = p.claim_rows;
+    const dim3 g1((unsigned)p.n1), b1(tms::kRowT), g2((unsigned)p.n2), b2(tms::kBlock);
+    if (p.ns == 1)
         hipLaunchKernelGGL((tms::spec_row_kernel<T, 1, tms::kRowT>), g1, b1, 0, stream, s);
-    else if (s.pv <= NSMAX / 2 * tms::kRowT)
+    else if (p.ns == NSMAX / 2)
         hipLaunchKernelGGL((tms::spec_row_kernel<T, NSMAX / 2, tms::kRowT>), g1, b1, 0, stream, s);
     else
         hipLaunchKernelGGL((tms::spec_row_kernel<T, NSMAX, tms::kRowT>), g1, b1, 0, stream, s);
-    if (wait)
+    if (p.wait)
         hipLaunchKernelGGL((tms::spec_resolve_kernel<T, true>), g2, b2, 0, stream, s);
     else
         hipLaunchKernelGGL((tms::spec_resolve_kernel<T, false>), g2, b2, 0, stream, s);

@@ -221,6 +221,7 @@ def test_spec_bonus_row_statistics_in_the_resolve(orc, sampler):
     ("bf16", 96, 66001, 2),                                               # places claimed in both launches
     ("f32", 72, 33001, 2),                                                # two parts a row, resident resolve
     ("f16", 2, 262145, 1),                                                # the ticket form of the resolve
+    ("f32", 1, 262145, 1), ("bf16", 1, 524289, 1),                        # one row's parts against an XCD's places
 ])
 def test_spec_rows_in_parts(orc, sampler, dtype, B, V, k):
     """Rows whose statistics several workgroups share, odd vocabularies (rows
