@@ -58,8 +58,8 @@ inline SpecPlan spec_plan(int B, int k, int V, int vec, int cap1, int cap2) {
         s.Lp = ((V + s.P - 1) / s.P + 7) / 8 * 8;
         s.P = (V + s.Lp - 1) / s.Lp;
     }
-    s.claim_parts = s.wait && B * s.P > cap2;
     s.n2 = (B + kSpecClaims - 1) / kSpecClaims * kSpecClaims * s.P;
+    s.claim_parts = s.wait && s.n2 > cap2;   // (an XCD holds the sequences of one residue)
     // The statistics: as few parts a row as registers allow, more where the
     // rows would leave compute units idle.  Where the grid takes more than
     // one round of the chip, the waiting resolve takes the bonus rows'

@@ -220,6 +220,7 @@ def test_spec_bonus_row_statistics_in_the_resolve(orc, sampler):
     ("f32", 2, 3, 2), ("bf16", 2, 7, 1), ("f16", 3, 9, 3),                # around one 16-byte vector
     ("bf16", 96, 66001, 2),                                               # places claimed in both launches
     ("f32", 72, 33001, 2),                                                # two parts a row, resident resolve
+    ("f32", 17, 98303, 1),                                                # a resolve resident but for the padding
     ("f16", 2, 262145, 1),                                                # the ticket form of the resolve
     ("f32", 1, 262145, 1), ("bf16", 1, 524289, 1),                        # one row's parts against an XCD's places
 ])

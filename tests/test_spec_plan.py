@@ -89,3 +89,13 @@ def test_a_rows_parts_leave_room(plans):
     least = -(-p["V"] // 32768)
     bad = p["S"] > np.maximum(least, CAP1 // XCDS // 4)
     assert not bad.any(), _first(p, bad)
+
+
+def test_places_are_claimed_where_the_grid_is_not_resident(plans):
+    """The grids are padded to whole counters: it is the padded grid whose
+    workgroups have to be resident at once, on every XCD."""
+    p = plans
+    bad = (p["S"] > 1) & (p["n1"] > CAP1) & (p["claim_rows"] == 0)
+    assert not bad.any(), _first(p, bad)
+    bad = (p["wait"] == 1) & (p["n2"] > CAP2) & (p["claim_parts"] == 0)
+    assert not bad.any(), _first(p, bad)
