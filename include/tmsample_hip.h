@@ -524,6 +524,10 @@ int tms_debug_philox(const uint32_t* in6, uint32_t* out4, int n, hipStream_t str
  * writing its half (counts has at least 7 entries). */
 int tms_debug_ordering(int trials, int32_t* counts);
 int tms_debug_exp(const double* in, double* out, int n, int which, hipStream_t stream);
+/* How often a workgroup of this context's tms_spec_verify calls looks for
+ * another's result before it forms that result itself (negative: the
+ * default; 0: at once).  The answers do not depend on it. */
+int tms_debug_spec_polls(tms_context* ctx, int polls);
 
 #ifdef __cplusplus
 }

@@ -14,6 +14,7 @@
 #include "tms_spec_plan.h"
 
 namespace tms {
+constexpr int kSpecPolls = 256;      // polls of a verify workgroup's wait for another
 constexpr int kPartWords = 3;      // u64 per part: weight sum, target sum, the bonus row's part max
 constexpr int kCounterStride = 64; // u32 between per-row arrival counters: one 256-byte line
                                    // each, so the rows' atomics do not queue on one line
@@ -45,6 +46,7 @@ struct tms_context {
     tms_spec_stat* spec_stats; // [max_batch][2 * kSpecMaxK + 1]
     uint64_t* spec_rparts;     // spec_rpart_words(): a row's part: its max word and its share of Z
     uint32_t* spec_claims;     // [2][8][kCounterStride] claim counters of the row kernel and the resolve
+    int spec_polls;            // polls of a verify workgroup's wait for another
     uint32_t* dlocks;          // [dense_slots] whole-row region locks
     int32_t* ov_n;             // [max_batch] history pre-pass: list lengths (-1: overflow)
     int32_t* ov_ids;           // [max_batch][TMS_HISTORY_MAX_IDS] listed ids

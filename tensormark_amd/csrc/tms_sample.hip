@@ -1358,6 +1358,7 @@ extern "C" int tms_create(int device, int max_batch, int max_vocab, tms_context*
     ctx->spec_stats = (tms_spec_stat*)(p + off_ss);
     ctx->spec_rparts = (uint64_t*)(p + off_sr);
     ctx->spec_claims = (uint32_t*)(p + off_sc);
+    ctx->spec_polls = tms::kSpecPolls;
     ctx->tlists = (uint64_t*)(p + off_tl);
     ctx->dlocks = (uint32_t*)(p + off_dq);
     ctx->ov_n = (int32_t*)(p + off_hn);

@@ -40,7 +40,7 @@ namespace tms {
 
 __constant__ double kSpecExpTab[64] = {TMS_EXP2_64THS};
 constexpr uint64_t kPartReady = 1ull << 63;   // published partial sum is complete
-constexpr int kPartPoll = 1 << 20;            // bound on the finisher's wait per part
+constexpr int kPartPoll = 1 << 20;            // bound on the finisher's wait per part, which has been stored
 
 constexpr int kRowW = kRowT / 64;
 
@@ -51,6 +51,13 @@ constexpr int kRowW = kRowT / 64;
 // workgroups that have still to start, which those rows' ends let in.
 // kSpecClaims counters, each with the rows (or sequences) of its residue,
 // share the traffic.  The last claim resets its counter.
+//
+// Other contexts' kernels may hold the places that the last workgroups need,
+// and wait themselves.  So no answer depends on a wait: a workgroup polls
+// `polls` times (some 0.2 ms, where a call takes 20 to 100 us); then it forms
+// a missing maximum from the logits itself, or leaves the draw to the
+// sequence's last workgroup, for which every sum is there.  The results are
+// the same whoever forms them.
 struct SArgs {
     const void* target;
     const void* draft;
@@ -71,6 +78,7 @@ struct SArgs {
     uint64_t* rparts;    // [B * (2k + 1)][S][2]: a part's max word and its share of Z
     uint32_t* claims;    // [2][kSpecClaims][kCounterStride]: row kernel, resolve
     bool claim_rows, claim_parts;   // the grid may not be resident at once
+    int polls;           // of a wait for another workgroup
 #ifdef TMS_TRACE
     uint64_t* trace;     // trace builds: 8 stamps per workgroup
 #endif
@@ -97,6 +105,7 @@ struct SpecLds {
     int stok[kSpecMaxK];
     double su[kSpecMaxK];
     int claim;
+    uint64_t late;       // the parts a wait ran out for
 };
 
 // This workgroup's place in a grid of kSpecClaims x n: (row, part) of rows
@@ -112,7 +121,7 @@ __device__ __forceinline__ void place(int S, bool claimed, uint32_t* counters, S
             L.claim = (int)m;
         }
         lds_sync();
-        n = L.claim;
+        n = __builtin_amdgcn_readfirstlane(L.claim);
     }
     row = n / S * kSpecClaims + c;
     part = n % S;
@@ -414,9 +423,13 @@ __device__ void accept_tests(const SArgs& a, int b, SpecLds& L, int& status, int
 // WAIT (up to kSpecParts parts of runs of at most kRunMax ids): every
 // workgroup keeps its part's weights in registers, reads every part's sums
 // (bounded wait), and the one whose part holds the draw's threshold locates
-// the token from its registers; the last reader (by a done counter) zeroes
-// the parts.  Otherwise the last arriver by ticket gathers the parts and
-// recomputes the weights of the part holding the threshold.
+// the token from its registers (from the logits again for a residual of no
+// mass, which is drawn by the target's weights).  One whose wait ran out says so and is gone.
+// The last of the P to count itself (each after its words are stored and its
+// loads returned) zeroes the parts, and locates the token if its workgroup is
+// gone, from that part's weights again.
+// Otherwise the last arriver by ticket gathers the parts and recomputes the
+// weights of the part holding the threshold.
 template <typename T, bool WAIT>
 __device__ void resolve_part(const SArgs& a, int b, int p, SpecLds& L) {
     const double* tab = L.tab;
@@ -458,7 +471,8 @@ __device__ void resolve_part(const SArgs& a, int b, int p, SpecLds& L) {
     __syncthreads();   // exp table in LDS
     const int lo = p * a.Lp, hi = min(a.V, lo + a.Lp);
     int64_t wsum = 0, tsum = 0;
-    int64_t wr[kRunMax], er[kRunMax];   // WAIT: the run's draw and target weights
+    int64_t wr[kRunMax];                // a run's weights
+    double mtu = mt;                    // the target row's maximum of v / T
     if constexpr (WAIT) {
         // a contiguous run of ids per thread, every load issued at once
         const int E = a.Lp / kBlock;   // a multiple of the vector width
@@ -491,7 +505,6 @@ __device__ void resolve_part(const SArgs& a, int b, int p, SpecLds& L) {
                 }
             }
         }
-        double mtu = mt;
         if (a.lazy && rej < 0) {
             // The bonus row's statistics (the row kernel left them): each
             // part's max of v / T and NaN / +inf flag, exchanged between the
@@ -511,20 +524,24 @@ __device__ void resolve_part(const SArgs& a, int b, int p, SpecLds& L) {
             pnf = block_or(pnf, misc);
             uint64_t* mw = a.parts + ((int64_t)b * kSpecParts + p) * kPartWords + 2;
             if (t == 0) st_agent(mw, kPartReady | ((uint64_t)pnf << 32) | okey(pm));
-            int bad = 0;
             uint32_t km = 0;
             int knf = 0;
-            if (t < a.P) {
-                const uint64_t* q = a.parts + ((int64_t)b * kSpecParts + t) * kPartWords + 2;
-                uint64_t h = 0;
-                for (int it = 0; it < kPartPoll; ++it) {
-                    h = ld_agent(q);
-                    if (h & kPartReady) break;
-                    __builtin_amdgcn_s_sleep(1);
+            if (t < 64) {
+                bool late = false;
+                if (t < a.P) {
+                    const uint64_t* q = a.parts + ((int64_t)b * kSpecParts + t) * kPartWords + 2;
+                    uint64_t h = 0;
+                    for (int it = 0; it < a.polls; ++it) {
+                        h = ld_agent(q);
+                        if (h & kPartReady) break;
+                        __builtin_amdgcn_s_sleep(1);
+                    }
+                    late = !(h & kPartReady);
+                    km = (uint32_t)h;
+                    knf = (int)((h >> 32) & 1u);
                 }
-                bad = (h & kPartReady) ? 0 : 1;
-                km = (uint32_t)h;
-                knf = (int)((h >> 32) & 1u);
+                const uint64_t all = __ballot(late);
+                if (t == 0) L.late = all;
             }
             // the bonus maxima's readers: the last zeroes the words and its
             // counter.  The waves' maxima meet in part_w, whose next writes
@@ -532,9 +549,9 @@ __device__ void resolve_part(const SArgs& a, int b, int p, SpecLds& L) {
             // the sums' own scratch.
             km = (uint32_t)wave_max_u64(km);
             if ((t & 63) == 0) part_w[t >> 6] = (int64_t)km;
-            bad = block_or(bad, misc);
             knf = block_or(knf, misc);
             if (t == 0) {
+                __builtin_amdgcn_s_waitcnt(0);   // this workgroup's word is stored
                 const uint32_t done = __hip_atomic_fetch_add(&a.tickets[b * kCounterStride + 1], 1u,
                                                              __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
                 misc[2] = done == (uint32_t)(a.P - 1) ? 1 : 0;
@@ -546,10 +563,26 @@ __device__ void resolve_part(const SArgs& a, int b, int p, SpecLds& L) {
                 if (t < a.P) st_agent(a.parts + ((int64_t)b * kSpecParts + t) * kPartWords + 2, (uint64_t)0);
                 if (t == 0) st_agent(&a.tickets[b * kCounterStride + 1], 0u);
             }
+            const uint64_t late = (uint64_t)readlane_i64((int64_t)L.late, 0);
+            if (late) {   // those parts' maxima, from the row
+                __syncthreads();
+                pm = -__builtin_huge_valf();
+                pnf = 0;
+                for (uint64_t m = late; m; m &= m - 1) {
+                    const int j0 = __builtin_ctzll(m) * a.Lp, j1 = min(a.V, j0 + a.Lp);
+#pragma unroll 1
+                    for (int id = j0 + t; id < j1; id += kBlock) {
+                        const float v = Elt<T>::scalar(rt + id);
+                        pnf |= (__builtin_isnan(v) || v == __builtin_huge_valf()) ? 1 : 0;
+                        pm = fmaxf(pm, scaled(v, temp));
+                    }
+                }
+                kmax = max(kmax, okey(block_max_f32(pm, L.shf)));
+                knf |= block_or(pnf, misc);
+            }
             const float gm = okey_inv(kmax);
             int st = TMS_ROW_OK;
-            if (bad) st = TMS_ROW_INTERNAL;
-            else if (knf) st = TMS_ROW_NONFINITE;
+            if (knf) st = TMS_ROW_NONFINITE;
             else if (gm == -__builtin_huge_valf()) st = TMS_ROW_ALL_MASKED;
             else if (gm == __builtin_huge_valf()) st = TMS_ROW_NONFINITE;
             if (st != TMS_ROW_OK) {
@@ -564,14 +597,13 @@ __device__ void resolve_part(const SArgs& a, int b, int p, SpecLds& L) {
         }
 #pragma unroll
         for (int j = 0; j < kRunMax; ++j) {
-            er[j] = 0;
             wr[j] = 0;
             if (r_lo + j < r_hi) {
                 const double etf = weight_f(xt[j], temp, mtu, tab);
-                er[j] = as_i64(etf);
-                wr[j] = rej < 0 ? er[j] : res(etf, weight_f(xd[j], temp, md, tab));
+                const int64_t et = as_i64(etf);
+                wr[j] = rej < 0 ? et : res(etf, weight_f(xd[j], temp, md, tab));
+                tsum += et;
             }
-            tsum += er[j];
             wsum += wr[j];
         }
     } else if (rej < 0) {
@@ -615,7 +647,7 @@ __device__ void resolve_part(const SArgs& a, int b, int p, SpecLds& L) {
     if (t < a.P) {
         uint64_t* q = a.parts + ((int64_t)b * kSpecParts + t) * kPartWords;
         uint64_t w = 0, u = 0;
-        for (int it = 0; it < kPartPoll; ++it) {
+        for (int it = 0; it < (WAIT ? a.polls : kPartPoll); ++it) {
             w = ld_agent(&q[0]);
             u = ld_agent(&q[1]);
             if ((w & kPartReady) && (u & kPartReady)) break;
@@ -629,34 +661,50 @@ __device__ void resolve_part(const SArgs& a, int b, int p, SpecLds& L) {
             st_agent(&q[1], (uint64_t)0);
         }
     }
-    timed_out = block_or(timed_out, misc);
+    uint64_t gone = 0;   // WAIT, in the last workgroup: the parts whose workgroup's wait ran out
     if constexpr (WAIT) {
-        // every word read: the last of the P readers (a relaxed counter; each
-        // adds after its loads returned) zeroes the parts and the counter
+        static_assert(kSpecParts <= 64, "the parts in one wave");
+        uint32_t* done = a.tickets + b * kCounterStride;
+        uint64_t* left = (uint64_t*)(done + 2);
+        const bool leave = __ballot(timed_out != 0) != 0;   // (the first wave)
         if (t == 0) {
-            const uint32_t done = __hip_atomic_fetch_add(&a.tickets[b * kCounterStride], 1u, __ATOMIC_RELAXED,
-                                                         __HIP_MEMORY_SCOPE_AGENT);
-            misc[1] = done == (uint32_t)(a.P - 1) ? 1 : 0;
+            if (leave) __hip_atomic_fetch_or(left, 1ull << p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            __builtin_amdgcn_s_waitcnt(0);
+            const uint32_t n = __hip_atomic_fetch_add(done, leave ? 0x10001u : 1u, __ATOMIC_RELAXED,
+                                                      __HIP_MEMORY_SCOPE_AGENT);
+            const bool last = (n & 0xFFFFu) == (uint32_t)(a.P - 1);
+            L.late = last && ((n >> 16) || leave) ? ld_agent(left) : 0ull;
+            misc[1] = last ? 1 : leave ? 2 : 0;
         }
         __syncthreads();
-        if (misc[1]) {
+        const int role = __builtin_amdgcn_readfirstlane(misc[1]);
+        if (role == 2) return;
+        gone = (uint64_t)readlane_i64((int64_t)L.late, 0);
+        if (role == 1) {
             if (t < a.P) {
                 uint64_t* q = a.parts + ((int64_t)b * kSpecParts + t) * kPartWords;
+                if (gone) {
+                    part_w[t] = (int64_t)(ld_agent(&q[0]) & ~kPartReady);
+                    part_t[t] = (int64_t)(ld_agent(&q[1]) & ~kPartReady);
+                }
                 st_agent(&q[0], (uint64_t)0);
                 st_agent(&q[1], (uint64_t)0);
             }
-            if (t == 0) st_agent(&a.tickets[b * kCounterStride], 0u);
+            if (t == 0) {
+                st_agent(done, 0u);
+                st_agent(left, (uint64_t)0);
+            }
+            if (gone) __syncthreads();
         }
-    }
-    SPEC_TR(4);
-    if (timed_out) {
-        if (t == 0 && (!WAIT || p == 0)) {
+    } else if (block_or(timed_out, misc)) {
+        if (t == 0) {
             a.out_acc[b] = 0;
             a.out_tok[b] = -1;
             a.out_status[b] = TMS_ROW_INTERNAL;
         }
         return;
     }
+    SPEC_TR(4);
     // The parts' sums across the lanes of each wave (P <= 64), by integer
     // scans: exact, so W, the threshold's part and the sum before it equal
     // the sequential sums.  Residual mass 0 (p_t <= p_d everywhere on the
@@ -680,31 +728,56 @@ __device__ void resolve_part(const SArgs& a, int b, int p, SpecLds& L) {
     const uint64_t over = __ballot(pl < a.P && sc > thr);
     const int ps = over ? __ffsll((unsigned long long)over) - 1 : a.P - 1;
     const int64_t base = ps > 0 ? readlane_i64(sc, ps - 1) : 0;
-    if (WAIT && ps != p) return;   // another workgroup holds the threshold's part
+    if (WAIT && ps != p && !((gone >> ps) & 1)) return;   // another workgroup holds the threshold's part
     SPEC_TR(6);
     // The part's weights, a contiguous run of ids per thread.
     const int plo = ps * a.Lp, phi = min(a.V, plo + a.Lp);
     const int E = WAIT ? a.Lp / kBlock : (phi - plo + kBlock - 1) / kBlock;
     const int my_lo = min(phi, plo + t * E), my_hi = min(phi, my_lo + E);
     auto w_at = [&](int id) -> int64_t {
-        const double et = weight_f(Elt<T>::scalar(rt + id), temp, mt, tab);
+        const double et = weight_f(Elt<T>::scalar(rt + id), temp, mtu, tab);
         if (use_t) return as_i64(et);
         return res(et, weight_f(Elt<T>::scalar(rd + id), temp, md, tab));
+    };
+    // The threads' sums `mine`, scanned; the thread that holds the threshold
+    // walks its run from the sum before it.
+    auto locate = [&](int64_t mine, auto&& walk) {
+        const int lane = t & 63, wv = t >> 6;
+        const int64_t inc = wave_incl_scan_i64(mine);
+        if (lane == 63) shl[wv] = inc;
+        __syncthreads();
+        SPEC_TR(5);
+        int64_t pre = base;
+        for (int i = 0; i < wv; ++i) pre += shl[i];
+        pre += inc - mine;
+        if (mine > 0 && pre <= thr && thr < pre + mine) {
+            a.out_acc[b] = acc;
+            a.out_tok[b] = walk(pre);
+            a.out_status[b] = TMS_ROW_OK;
+        }
+    };
+    auto walk_ids = [&](int64_t sum) {
+#pragma unroll 1
+        for (int id = my_lo; id < my_hi; ++id) {
+            sum += w_at(id);
+            if (sum > thr) return id;
+        }
+        return my_hi - 1;
     };
     // Runs of up to kRunMax ids: every load issued at once (clamped
     // addresses), the weights kept in registers for the scan and the search;
     // longer runs walk the ids one by one.  WAIT: this workgroup's own run
-    // weights, still in registers.
-    const bool cached = WAIT || E <= kRunMax;
-    int64_t wc[kRunMax];
+    // weights, still in registers; others one by one.
+    const bool cached = WAIT ? ps == p && (rej < 0 || !use_t) : E <= kRunMax;
     int64_t mine = 0;
-    if constexpr (WAIT) {
-#pragma unroll
-        for (int j = 0; j < kRunMax; ++j) {
-            wc[j] = use_t ? er[j] : wr[j];
-            mine += wc[j];
-        }
-    } else if (cached) {
+    if (!cached) {
+#pragma unroll 1
+        for (int id = my_lo; id < my_hi; ++id) mine += w_at(id);
+        SPEC_TR(7);
+        locate(mine, walk_ids);
+        return;
+    }
+    if constexpr (!WAIT) {
         float xt[kRunMax], xd[kRunMax];
 #pragma unroll
         for (int j = 0; j < kRunMax; ++j) {
@@ -714,49 +787,29 @@ __device__ void resolve_part(const SArgs& a, int b, int p, SpecLds& L) {
         }
 #pragma unroll
         for (int j = 0; j < kRunMax; ++j) {
-            wc[j] = 0;
+            wr[j] = 0;
             if (my_lo + j < my_hi) {
                 const double et = weight_f(xt[j], temp, mt, tab);
-                wc[j] = use_t ? as_i64(et) : res(et, weight_f(xd[j], temp, md, tab));
+                wr[j] = use_t ? as_i64(et) : res(et, weight_f(xd[j], temp, md, tab));
             }
-            mine += wc[j];
         }
-    } else {
-        for (int id = my_lo; id < my_hi; ++id) mine += w_at(id);
     }
-    SPEC_TR(7);
-    // Exclusive scan of the threads' sums.
-    const int lane = t & 63, wv = t >> 6;
-    const int64_t inc = wave_incl_scan_i64(mine);
-    if (lane == 63) shl[wv] = inc;
-    __syncthreads();
-    SPEC_TR(5);
-    int64_t pre = base;
-    for (int i = 0; i < wv; ++i) pre += shl[i];
-    pre += inc - mine;
-    if (mine > 0 && pre <= thr && thr < pre + mine) {
-        int64_t acc_w = pre;
-        int tok = my_hi - 1;
-        if (cached) {
-            bool found = false;
 #pragma unroll
-            for (int j = 0; j < kRunMax; ++j) {
-                acc_w += wc[j];
-                if (!found && my_lo + j < my_hi && acc_w > thr) {
-                    tok = my_lo + j;
-                    found = true;
-                }
-            }
-        } else {
-            for (int id = my_lo; id < my_hi; ++id) {
-                acc_w += w_at(id);
-                if (acc_w > thr) { tok = id; break; }
+    for (int j = 0; j < kRunMax; ++j) mine += wr[j];
+    SPEC_TR(7);
+    locate(mine, [&](int64_t sum) {
+        int tok = my_hi - 1;
+        bool found = false;
+#pragma unroll
+        for (int j = 0; j < kRunMax; ++j) {
+            sum += wr[j];
+            if (!found && my_lo + j < my_hi && sum > thr) {
+                tok = my_lo + j;
+                found = true;
             }
         }
-        a.out_acc[b] = acc;
-        a.out_tok[b] = tok;
-        a.out_status[b] = TMS_ROW_OK;
-    }
+        return tok;
+    });
 }
 
 
@@ -869,42 +922,65 @@ void spec_row_kernel(SArgs a) {
             nf |= L.misc[j];
         }
     }
-    int bad = 0;
     uint64_t* rp = a.rparts + ((int64_t)b * (2 * a.k + 1) + i) * a.S * 2;
     if (a.S > 1) {   // the row's, from every part's word
         if (t == 0) st_agent(rp + 2 * p, kPartReady | ((uint64_t)nf << 32) | okey(mx));
         if (t < 64) {
-            uint32_t km = 0;
-            for (int j = t; j < a.S; j += 64) {
+            uint32_t km = okey(mx);
+            bool late = false;
+            if (t < a.S && t != p) {
                 uint64_t h = 0;
-                for (int it = 0; it < kPartPoll; ++it) {
-                    h = ld_agent(rp + 2 * j);
+                for (int it = 0; it < a.polls; ++it) {
+                    h = ld_agent(rp + 2 * t);
                     if (h & kPartReady) break;
                     __builtin_amdgcn_s_sleep(1);
                 }
-                bad |= (h & kPartReady) ? 0 : 1;
+                late = !(h & kPartReady);
                 nf |= (int)((h >> 32) & 1u);
                 km = max(km, (uint32_t)h);
             }
             km = (uint32_t)wave_max_u64(km);
             nf = __any(nf) ? 1 : 0;
-            bad = __any(bad) ? 1 : 0;
+            const uint64_t all = __ballot(late);
             if (t == 0) {
                 L.stok[0] = (int)km;
-                L.stok[1] = nf | bad << 1;
+                L.stok[1] = nf;
+                L.late = all;
             }
         }
         lds_sync();
         mx = okey_inv((uint32_t)L.stok[0]);
-        nf = L.stok[1] & 1;
-        bad = L.stok[1] >> 1;
+        nf = L.stok[1];
+        const uint64_t late = (uint64_t)readlane_i64((int64_t)L.late, 0);
+        if (late) {   // those parts' maxima, from the row
+            for (uint64_t m = late; m; m &= m - 1) {
+                const int j0 = __builtin_ctzll(m) * a.pv * VEC, j1 = min(j0 + a.pv * VEC, V);
+#pragma unroll 1
+                for (int id = j0 + t; id < j1; id += NT) {
+                    const float v = Elt<T>::scalar(row + id);
+                    nf |= __builtin_amdgcn_class(v, 0x203);   // NaN or +inf
+                    mx = fmaxf(mx, v);
+                }
+            }
+            mx = wave_max_f32(mx);
+            nf = __any(nf) ? 1 : 0;
+            if ((t & 63) == 0) {
+                L.shf[t >> 6] = mx;
+                L.misc[t >> 6] = nf;
+            }
+            lds_sync();
+#pragma unroll
+            for (int j = 0; j < NW; ++j) {
+                mx = fmaxf(mx, L.shf[j]);
+                nf |= L.misc[j];
+            }
+        }
     }
     const float temp = a.params[b].temperature;
     const bool div = temp != 1.0f;
     mx = scaled(mx, temp);
     int st = TMS_ROW_OK;
-    if (bad) st = TMS_ROW_INTERNAL;
-    else if (nf) st = TMS_ROW_NONFINITE;
+    if (nf) st = TMS_ROW_NONFINITE;
     else if (mx == -__builtin_huge_valf()) st = TMS_ROW_ALL_MASKED;
     else if (mx == __builtin_huge_valf()) st = TMS_ROW_NONFINITE;
     const double md = (double)mx;
@@ -984,6 +1060,13 @@ static int launch_verify(tms::SArgs s, hipStream_t stream) {
     return hipGetLastError() == hipSuccess ? TMS_OK : TMS_ERR_HIP;
 }
 
+// Test hook: polls of a wait for another workgroup (negative: the default).
+extern "C" int tms_debug_spec_polls(tms_context* ctx, int polls) {
+    if (!ctx) return TMS_ERR_INVALID_ARG;
+    ctx->spec_polls = polls < 0 ? tms::kSpecPolls : polls;
+    return TMS_OK;
+}
+
 extern "C" int tms_spec_verify(tms_context* ctx, const tms_spec_args* a, hipStream_t stream) {
     if (!ctx || !a || !a->target_logits || !a->draft_logits || !a->draft_tokens || !a->params ||
         !a->out_accepted || !a->out_token || !a->out_status)
@@ -1021,6 +1104,7 @@ extern "C" int tms_spec_verify(tms_context* ctx, const tms_spec_args* a, hipStre
 #endif
     s.rparts = ctx->spec_rparts;
     s.claims = ctx->spec_claims;
+    s.polls = ctx->spec_polls;
     switch (a->dtype) {
         case TMS_DTYPE_F32: return launch_verify<float>(s, stream);
         case TMS_DTYPE_F16: return launch_verify<_Float16>(s, stream);

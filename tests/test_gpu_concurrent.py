@@ -1,12 +1,14 @@
 """The residency-dependent kernels beside concurrent GPU work.
 
-The wide top-k kernel and the verify's waiting resolve are chosen only when
-their grid fits the device at once; their workgroups wait on each other with
-bounded waits.  Here they run on one stream while a second stream (default
-priority) runs large matrix multiplications that hold compute units, so some
-of their workgroups start late.  Every row must equal the oracle's answer or
-report TMS_ROW_INTERNAL; after an internal error a workspace reset and a
-repeat give the oracle's answer.  No row may carry a wrong token."""
+The wide top-k kernel is chosen only when its grid fits the device at once;
+its workgroups and the verify's wait on each other with bounded waits.  Here
+they run on one stream while a second stream (default priority) runs large
+matrix multiplications that hold compute units, so some of their workgroups
+start late.  Every row must equal the oracle's answer or report
+TMS_ROW_INTERNAL; after an internal error a workspace reset and a repeat give
+the oracle's answer.  No row may carry a wrong token.  A verify whose waits run
+out works the missing parts out itself, so contexts that verify at once, whose
+waiting workgroups hold each other's places, answer every sequence."""
 from __future__ import annotations
 
 import numpy as np
@@ -115,3 +117,40 @@ def test_verify_beside_a_busy_stream(sampler, orc):
     torch.cuda.synchronize()
     for b, (wst, wacc, wtok) in enumerate(want):
         assert (o["status"][b].item(), o["accepted"][b].item(), o["token"][b].item()) == (wst, wacc, wtok), b
+
+
+def test_contexts_verify_at_once(orc):
+    """Four contexts on four streams: one sequence's rows in parts, and grids
+    that take their places in order."""
+    import torch
+
+    from tensormark_amd import Sampler
+    from tests.helpers import params_array
+    from tests.test_gpu_spec import philox_words, widen
+
+    rng = np.random.default_rng(17)
+    jobs = []
+    for B, k, V in ((1, 1, 256000), (1, 1, 256000), (40, 2, 66001), (40, 2, 66001)):
+        target = rng.standard_normal((B, k + 1, V), dtype=np.float32) * 2.0
+        draft = target[:, :k] + 0.7 * rng.standard_normal((B, k, V), dtype=np.float32)
+        tokens = workloads.softmax_draws(rng, draft).astype(np.int32)
+        p = params_array(B, temperature=0.9, seed=np.arange(B) + V)
+        words = philox_words(orc, p, k)
+        tg, dr = widen(target, "bf16"), widen(draft, "bf16")
+        want = [orc.spec_verify_seq(tg[b], dr[b], tokens[b], 0.9, words[b]) for b in range(B)]
+        s = Sampler(max_batch=B, max_vocab=V)
+        jobs.append((s, torch.cuda.Stream(),
+                     (_dev(workloads.to_bf16_bits(target), torch.bfloat16),
+                      _dev(workloads.to_bf16_bits(draft), torch.bfloat16), _dev(tokens), s.params_tensor(p)), want))
+    torch.cuda.synchronize()
+    outs = []
+    for _ in range(8):
+        for i, (s, stream, args, _) in enumerate(jobs):
+            with torch.cuda.stream(stream):
+                outs.append((i, {n: v.clone() for n, v in s.spec_verify(*args).items()}))
+    torch.cuda.synchronize()
+    for i, o in outs:
+        got = list(zip(*(o[n].tolist() for n in ("status", "accepted", "token"))))
+        assert got == jobs[i][3], i
+    for s, *_ in jobs:
+        s.close()

@@ -246,3 +246,57 @@ def test_spec_rows_in_parts(orc, sampler, dtype, B, V, k):
     for _ in range(2):
         gpu = run_spec(sampler, target, draft, tokens, params, dtype=dtype)
         check_spec(orc, gpu, target, draft, tokens, params, words, dtype)
+
+
+@pytest.mark.parametrize("dtype,B,V,k", [
+    ("bf16", 1, 151937, 4), ("f32", 1, 40000, 1),      # a row's parts, a resolve in parts of 8 ids a thread
+    ("f32", 32, 4001, 8), ("bf16", 40, 131073, 3),     # bonus rows in the resolve, one and several parts a row
+])
+def test_spec_answers_do_not_depend_on_the_waits(orc, dtype, B, V, k):
+    """Workgroups that never wait for each other, or hardly: each forms the
+    maxima it misses itself, and the sequence's last workgroup draws for those
+    that are gone.  Rejected and accepted sequences, bonus rows with a NaN and
+    with nothing allowed; a call with the default waits after them finds the
+    shared words as it should."""
+    from tensormark_amd import Sampler
+
+    rng = np.random.default_rng(V + k)
+    target = rng.standard_normal((B, k + 1, V), dtype=np.float32) * 2.0
+    draft = target[:, :k] + 0.7 * rng.standard_normal((B, k, V), dtype=np.float32)
+    draft[::2] = target[::2, :k]                      # every draft accepted
+    tokens = workloads.softmax_draws(rng, draft)
+    params = params_array(B, temperature=1.0, seed=np.arange(B) + 11)
+    params["temperature"] = rng.choice([0.7, 1.0, 1.3], size=B)
+    if B > 4:
+        target[2, k, V - 1] = np.nan
+        target[4, k, :] = -np.inf
+    words = philox_words(orc, params, k)
+    s = Sampler(max_batch=B, max_vocab=V)
+    try:
+        for polls in (0, 1, 0, 2, -1):
+            assert s.lib.tms_debug_spec_polls(s.handle, polls) == 0
+            gpu = run_spec(s, target, draft, tokens, params, dtype=dtype)
+            check_spec(orc, gpu, target, draft, tokens, params, words, dtype)
+    finally:
+        s.close()
+
+
+def test_spec_residual_without_mass(orc, sampler):
+    """A rejection whose residual rounds to nothing: the draft's token is one
+    float less likely in the target, and no other id gains 2^-45.  The draw is
+    from the target's weights."""
+    rng = np.random.default_rng(5)
+    B, k, V = 4, 2, 9000
+    target = rng.normal(0.0, 1.0, (B, k + 1, V)).astype(np.float32)
+    draft = target[:, :k].copy()
+    tokens = np.argmax(np.abs(target[:, :k] + 1.0) < 0.01, axis=2).astype(np.int32)
+    for b in range(B):
+        for i in range(k):
+            x = tokens[b, i]
+            draft[b, i, x] = np.nextafter(draft[b, i, x], np.float32(np.inf))
+    params = params_array(B, temperature=1.0)
+    words = np.full((B, k + 1, 2), 0xFFFFFFFF, np.uint32)   # the accept tests' uniforms: next to 1
+    words[:, k] = rng.integers(0, 2**32, size=(B, 2), dtype=np.uint64)
+    gpu = run_spec(sampler, target, draft, tokens, params, draws=words)
+    check_spec(orc, gpu, target, draft, tokens, params, words)
+    assert (gpu["status"] == 0).all() and (gpu["accepted"] == 0).all()
