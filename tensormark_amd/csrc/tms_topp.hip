@@ -490,7 +490,8 @@ __device__ __forceinline__ bool plan(const KArgs& a, Row& R, Lds& L) {
         const bool in = d >= -41.5;
         L.cw[t] = in ? exp_span(fmax(d, -42.0), L.tab) : 0.0;
         L.shift[t] = in ? R.top - topp_bucket(cm) : kHistBuckets;
-        if (in && !(L.head[t] >> 32)) L.lost = 1;
+        // (entries that a record lost may lie above its maximum, and above the row's)
+        if (!(L.head[t] >> 32)) L.lost = 1;
     }
     lds_sync();
     double m = 0.0;

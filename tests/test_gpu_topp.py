@@ -126,3 +126,24 @@ def test_calls_in_a_row_and_a_captured_graph(ctx):
         again = ctx.sample(x.flip(0).contiguous(), p)   # the program's own work between replays
         torch.cuda.synchronize()
         assert int(again["status"].abs().sum()) == 0
+
+
+@pytest.mark.parametrize("high", [0, 1, 2000])
+def test_more_penalised_ids_than_a_record_holds(ctx, orc, high):
+    """3000 of the first chunk's ids in the window, the only ones allowed there:
+    a record holds 1024 of them, in any order.  None, one or most of them are
+    among the row's likely ids."""
+    B, V = 16, 20000
+    rng = np.random.default_rng(high)
+    x = rng.normal(0.0, 0.5, (B, V)).astype(np.float32)
+    x[:, :8192] = -200.0
+    recent = np.stack([rng.choice(8192, 3000, replace=False) for _ in range(B)])
+    for b in range(B):
+        x[b, rng.choice(recent[b], high, replace=False)] = 10.0 if high == 1 else 1.0
+    allowed = np.ones((B, (V + 31) // 32 * 32), bool)
+    allowed[:, V:] = False
+    allowed[:, :8192] = False
+    allowed[np.arange(B)[:, None], recent] = True
+    mask = np.packbits(allowed, axis=1, bitorder="little").view(np.uint32)
+    p = params_array(B, top_k=0, temperature=1.0, top_p=0.9, repeat_penalty=1.1, repeat_last_n=4000, seed=np.arange(B))
+    check(run_gpu(ctx, x, p, recent=recent, mask=mask), orc.sample_batch(x, p, recent=recent, mask=mask))
