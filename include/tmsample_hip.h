@@ -242,8 +242,12 @@ const char* tms_status_string(int code);
 
 /*
  * Create a context on `device` for batches up to max_batch rows of up to
- * max_vocab ids.  Allocates the workspace (per-row counters and candidate
- * lists) once; the sampling calls allocate nothing.  A context serves one
+ * max_vocab ids.  Allocates the workspace once; the sampling calls allocate
+ * nothing.  Its largest parts are for 256 rows at most, also where max_batch
+ * is larger: a row sampled whole takes 16 bytes an id of max_vocab, and one of
+ * the whole-vocabulary kernel 52 KiB a 16384 ids (of at most 262144) and 80
+ * KiB.  The rest is some 40 KiB a row, and 5 KiB a row and 16384 ids.
+ * tms_workspace_bytes has the sum.  A context serves one
  * stream at a time: concurrent calls on one context race on its workspace.
  * Replaces the library-owned state the reference keeps in its Metal token
  * slots (tensormark/metal.h:3191-3228).

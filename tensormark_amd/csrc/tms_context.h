@@ -51,11 +51,13 @@ struct tms_context {
     int32_t* ov_n;             // [max_batch] history pre-pass: list lengths (-1: overflow)
     int32_t* ov_ids;           // [max_batch][TMS_HISTORY_MAX_IDS] listed ids
     float* ov_vals;            // [max_batch][TMS_HISTORY_MAX_IDS] their final values
-    uint64_t* hist;            // the rows' chunk records (tms_topp.h)
+    uint64_t* hist;            // [topp_slots] rows' chunk records (tms_topp.h)
+    uint32_t* topp_locks;      // [topp_slots] locks of those
+    int topp_slots;            // min(max_batch, kToppSlotsMax)
     uint32_t* topp_ctl;        // [max_batch][kToppCtl] row states and shared words
     uint32_t* topp_any;        // the last call that left a row to the second launch
     uint32_t topp_calls;       // calls so far, that word's values
-    uint64_t* topp_items;      // [max_batch][kToppRanges][kToppItemWords]
+    uint64_t* topp_items;      // [topp_slots][kToppRanges][kToppItemWords]
     uint64_t* dense;           // [dense_slots][2 * max_vocab] the whole-row path (separate allocation)
     int dense_slots;           // min(max_batch, kDenseSlotsMax) regions, each taken by a lock
     size_t dense_bytes;        // of `dense` with hist, topp_items and topp_ctl behind it

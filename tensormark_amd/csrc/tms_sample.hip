@@ -1318,7 +1318,8 @@ extern "C" int tms_create(int device, int max_batch, int max_vocab, tms_context*
     const size_t off_tl = off_sc + 2 * tms::kSpecClaims * tms::kCounterStride * sizeof(uint32_t);
     const size_t tl_chunks = (size_t)std::min(ctx->max_chunks, tms::kWideMaxChunksHost);
     const size_t off_dq = off_tl + nb * tl_chunks * tms::kWideListStride * sizeof(uint64_t);
-    const size_t off_hn = off_dq + 256 * (((size_t)tms::kDenseSlotsMax * sizeof(uint32_t) + 255) / 256);
+    const size_t off_tk = off_dq + 256 * (((size_t)tms::kDenseSlotsMax * sizeof(uint32_t) + 255) / 256);
+    const size_t off_hn = off_tk + 256 * (((size_t)tms::kToppSlotsMax * sizeof(uint32_t) + 255) / 256);
     const size_t off_hi = off_hn + 256 * ((nb * sizeof(int32_t) + 255) / 256);
     const size_t off_hv = off_hi + nb * tms::kHistMax * sizeof(int32_t);
     ctx->bytes = off_hv + nb * tms::kHistMax * sizeof(float);
@@ -1330,11 +1331,13 @@ extern "C" int tms_create(int device, int max_batch, int max_vocab, tms_context*
     // The whole-row path's region: never read before it is written, so not
     // cleared.
     ctx->dense_slots = std::min(max_batch, tms::kDenseSlotsMax);
-    // With it, the second launch's records (tms_topp.h), likewise written
-    // before they are read.
+    // With it, the second launch's records and items (tms_topp.h), likewise
+    // written before they are read: 0.93 MB a slot of 256,000 ids, for up to
+    // 256 rows (larger batches share them), and 256 bytes a row.
+    ctx->topp_slots = std::min(max_batch, tms::kToppSlotsMax);
     const size_t dense_words = (size_t)ctx->dense_slots * 2 * (size_t)max_vocab;
-    const size_t hist_words = tms::topp_hist_words(nb, max_vocab);
-    const size_t item_words = nb * tms::kToppRanges * tms::kToppItemWords;
+    const size_t hist_words = tms::topp_hist_words((size_t)ctx->topp_slots, max_vocab);
+    const size_t item_words = (size_t)ctx->topp_slots * tms::kToppRanges * tms::kToppItemWords;
     const size_t off_hw = (dense_words + 31) / 32 * 32;
     const size_t off_iw = off_hw + hist_words;
     const size_t off_cw = off_iw + item_words;
@@ -1361,6 +1364,7 @@ extern "C" int tms_create(int device, int max_batch, int max_vocab, tms_context*
     ctx->spec_polls = tms::kSpecPolls;
     ctx->tlists = (uint64_t*)(p + off_tl);
     ctx->dlocks = (uint32_t*)(p + off_dq);
+    ctx->topp_locks = (uint32_t*)(p + off_tk);
     ctx->ov_n = (int32_t*)(p + off_hn);
     ctx->ov_ids = (int32_t*)(p + off_hi);
     ctx->ov_vals = (float*)(p + off_hv);
@@ -1430,6 +1434,8 @@ struct SampleWs {
     int32_t* ov_ids;
     float* ov_vals;
     uint64_t* hist = nullptr;        // tms_topp.h (contexts only)
+    uint32_t* topp_locks = nullptr;
+    int topp_slots = 0;
     uint32_t* topp_ctl = nullptr;
     uint32_t* topp_any = nullptr;
     uint32_t topp_call = 0;
@@ -1492,6 +1498,8 @@ static int sample_launch(const SampleWs& w, const tms_sample_args* a, hipStream_
     // Calls without the top-k promise: dense top-p rows by a second launch.
     if (a->row_kinds != TMS_ROWS_TOPK && w.hist && a->vocab <= tms::kToppMaxVocab) {
         k.hist = w.hist;
+        k.topp_locks = w.topp_locks;
+        k.topp_slots = w.topp_slots;
         k.topp_ctl = w.topp_ctl;
         k.topp_any = w.topp_any;
         k.topp_call = w.topp_call;
@@ -1588,6 +1596,8 @@ extern "C" int tms_sample_batch(tms_context* ctx, const tms_sample_args* a, hipS
     w.ov_ids = ctx->ov_ids;
     w.ov_vals = ctx->ov_vals;
     w.hist = ctx->hist;
+    w.topp_locks = ctx->topp_locks;
+    w.topp_slots = ctx->topp_slots;
     w.topp_ctl = ctx->topp_ctl;
     w.topp_any = ctx->topp_any;
     w.topp_call = ++ctx->topp_calls;

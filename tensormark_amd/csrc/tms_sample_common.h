@@ -93,11 +93,13 @@ struct KArgs {
                            // `n_recent` its id lists (n_recent -1: the row overflowed);
                            // null when the call has no pre-pass
     // tms_topp.h, for calls whose dense top-p rows a second launch samples
-    uint64_t* hist;        // the rows' chunk records, written and read by that launch
+    uint64_t* hist;        // [topp_slots] rows' chunk records, written and read by that launch
+    uint32_t* topp_locks;  // [topp_slots]: 1 while a workgroup has the slot, for calls that leave more rows
+    int topp_slots;
     uint32_t* topp_ctl;    // [B][kToppCtl]: word 0 the row's state, then its workgroups' shared words
     uint32_t* topp_any;    // topp_call once the call has left a row to that launch
     uint32_t topp_call;
-    uint64_t* topp_items;  // [B][kToppRanges][kToppItemWords]
+    uint64_t* topp_items;  // [topp_slots][kToppRanges][kToppItemWords]
 #ifdef TMS_TRACE
     uint64_t* trace;
 #endif

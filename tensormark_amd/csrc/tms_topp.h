@@ -33,10 +33,14 @@ constexpr int kHistHead = kHistExt + kHistExtra;
 constexpr int kHistId = kHistHead + 2;
 static_assert(kHistIds + kHistExtra < 65536, "16-bit ids of a chunk");
 constexpr int hist_words(int chunk_ids) { return kHistId + chunk_ids / 4 + 2; }
-// Rows in small chunks at most, so that their records fit those of a whole
-// batch in large ones.
+// Slots of records and items in a workspace, at most: as many as workgroups of
+// that kernel run at once, one a CU.  A row of 256,000 ids takes 0.93 MB.
+constexpr int kToppSlotsMax = 256;
+// Rows in small chunks at most, so that their records fit those of as many
+// slots in large ones.
 constexpr int kHistSmallRows = 32;
 inline size_t topp_hist_words(size_t rows, int vocab) {
+    if (vocab > kToppMaxVocab) vocab = kToppMaxVocab;
     const size_t large = rows * (size_t)((vocab + kHistIds - 1) / kHistIds) * hist_words(kHistIds);
     const size_t few = rows < (size_t)kHistSmallRows ? rows : (size_t)kHistSmallRows;
     const size_t small = few * (size_t)((vocab + kHistIdsSmall - 1) / kHistIdsSmall) * hist_words(kHistIdsSmall);

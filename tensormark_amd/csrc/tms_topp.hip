@@ -36,6 +36,11 @@
 // in all, help them.  A chunk or a range is claimed by an atomic counter, so no
 // workgroup waits for one that has not started: whoever runs takes what is
 // left.
+//
+// A row's records and items are a slot of the workspace: the row's place among
+// the call's rows while those have a slot each.  More rows than slots (as many
+// as CUs, each of which holds one workgroup) take theirs by a lock and give
+// them back, and have no helpers, which could still be reading one.
 
 #include "tms_dense.h"
 #include "tms_topp.h"
@@ -107,7 +112,7 @@ struct Lds {
 
 // What every workgroup of a row knows after plan().
 struct Row {
-    int row, V, K, S, CE, words;   // CE ids a chunk, `words` a record
+    int row, slot, V, K, S, CE, words;   // CE ids a chunk, `words` a record
     float mx;        // the row's maximum of lg
     int top;         // its bucket
     int n;           // entries within the histogram's span
@@ -207,7 +212,7 @@ __device__ __forceinline__ int block_min(int v, Lds& L) {   // v >= 0
 template <typename T, int U, typename F>
 __device__ __forceinline__ int fetch(const KArgs& a, const Row& R, int3 j0, int3 j1, int nI, int most, Lds& L, F&& put) {
     const int t = threadIdx.x;
-    const uint64_t* rec = a.hist + (int64_t)R.row * R.S * R.words;
+    const uint64_t* rec = a.hist + (int64_t)R.slot * R.S * R.words;
     const T* base = (const T*)a.logits + (int64_t)R.row * a.row_stride;
     if (t < 64) {   // the runs, in one wave
         int len = 0, src = 0;
@@ -279,7 +284,7 @@ __device__ __forceinline__ void record(const KArgs& a, const Row& R, const tms_r
     const int e0 = c * R.CE, len = min(R.CE, R.V - e0);
     const T* base = (const T*)a.logits + (int64_t)R.row * a.row_stride + e0;
     const uint32_t* mrow = a.mask + (int64_t)R.row * a.mask_stride;
-    uint64_t* rec = a.hist + ((int64_t)R.row * R.S + c) * R.words;
+    uint64_t* rec = a.hist + ((int64_t)R.slot * R.S + c) * R.words;
     const int nv = len / VEC;   // whole vectors; the row's last ids one by one
     uint4 q[NVT];
     uint32_t mw[NVT];
@@ -473,7 +478,7 @@ __device__ __forceinline__ bool describe(const KArgs& a, int row, const tms_row_
 // workgroup of the row.
 __device__ __forceinline__ bool plan(const KArgs& a, Row& R, Lds& L) {
     const int t = threadIdx.x;
-    const uint64_t* rec = a.hist + (int64_t)R.row * R.S * R.words;
+    const uint64_t* rec = a.hist + (int64_t)R.slot * R.S * R.words;
     if (t < a.S) L.head[t] = ld_agent(&rec[(int64_t)t * R.words + kHistHead]);
     if (t == 0) L.lost = 0;
     lds_sync();
@@ -1229,7 +1234,7 @@ template <typename T>
 __device__ __forceinline__ int exact_keep(const KArgs& a, const Row& R, bool leader, Lds& L) {
     const int t = threadIdx.x;
     uint32_t* ctl = a.topp_ctl + (int64_t)R.row * kToppCtl;
-    uint64_t* items = a.topp_items + (int64_t)R.row * kToppRanges * kToppItemWords;
+    uint64_t* items = a.topp_items + (int64_t)R.slot * kToppRanges * kToppItemWords;
     // Ranges of at most kRange entries: whole buckets, about Q entries each.
     int big = t < kHistBuckets - 1 ? L.pc[t + 1] - L.pc[t] : 0;
     big = kRange - block_min(kRange - min(big, kRange), L);
@@ -1440,6 +1445,18 @@ __device__ __forceinline__ void records(const KArgs& a, const Row& R, const tms_
     }
 }
 
+// The rows before `row` that the general kernel left to this launch.
+__device__ __forceinline__ int rows_before(const KArgs& a, int row, Lds& L) {
+    int n = 0;
+    for (int b0 = 0; b0 < row; b0 += kT) {
+        const int b = b0 + (int)threadIdx.x;
+        int c;
+        excl_i(b < row && a.topp_ctl[(int64_t)b * kToppCtl] != TOPP_NONE ? 1 : 0, c, L);
+        n += c;
+    }
+    return n;
+}
+
 // Workgroup g takes the g-th of the rows, if there are so many; the others
 // help: with a row's records, then with a top_p = 1 row's ranges.
 template <typename T>
@@ -1452,51 +1469,61 @@ __global__ __launch_bounds__(kT) void topp_kernel(KArgs a, int B) {
     int n, ne;
     int row = pick_row(a, B, g, false, n, L);
     if (row < 0) return;
-    const bool leader = g < n;
+    const bool leader = g < n, shared = n > a.topp_slots;
+    if (shared && !leader) return;
     if (t < 64) L.tab[t] = kExpTab[t];
     // state words and parameters were written before this launch
     Row R;
-    bool whole = false;
+    R.slot = g % n;   // pick_row's row
+    if (shared) {
+        if (t == 0) L.misc[6] = take_dense_slot(a.topp_locks, a.topp_slots, g);
+        lds_sync();
+        R.slot = uni(L.misc[6]);
+        lds_sync();
+    }
+    bool whole = R.slot < 0;
     int how = SEL_WHOLE, tok = -1, rank = 0;
-    for (int turn = leader ? 1 : 0; turn < 2; ++turn) {
+    for (int turn = leader ? 1 : 0; turn < 2 && !whole; ++turn) {
         if (!leader && turn == 1) {
             row = pick_row(a, B, g - n, true, ne, L);
             if (row < 0) return;
+            R.slot = rows_before(a, row, L);
         }
         const tms_row_params P = a.params[row];
         uint32_t* ctl = a.topp_ctl + (int64_t)row * kToppCtl;
         whole = ctl[kCtlState] == TOPP_WHOLE || !describe(a, row, P, R);
         if (!whole) records<T>(a, R, P, ctl, L);
-        if (turn == 0) continue;
+        if (turn == 0) {
+            whole = false;
+            continue;
+        }
         if (!whole) whole = !wait_ge(&ctl[kCtlChunks], (uint32_t)R.S, kPollCap, L) || !plan(a, R, L);
     }
     const tms_row_params P = a.params[row];
-    if (!whole && R.mx == __builtin_huge_valf()) {
-        // v / T overflowed (the reference's maximum is +inf)
-        if (leader) write_row_error(a, row, TMS_ROW_NONFINITE);
-        return;
-    }
-    if (!whole && R.K < R.n) whole = true;
-    if (!whole && leader) {
+    const bool inf = !whole && R.mx == __builtin_huge_valf();   // v / T overflowed (the reference's maximum is +inf)
+    if (!whole && !inf && R.K < R.n) whole = true;
+    if (!whole && !inf && leader) {
         how = select<T>(a, P, R, L, tok, rank);
         whole = how == SEL_WHOLE;
         lds_sync();
     }
-    if (!leader && whole) return;
-    if (!whole && (!leader || how == SEL_EXACT)) {
+    if (!whole && !inf && (!leader || how == SEL_EXACT)) {
         const int keep = exact_keep<T>(a, R, leader, L);
-        if (!leader) return;
-        if (keep >= 2 && rank < keep - 1) {
-            if (t == 0) {
-                a.out_tokens[row] = tok;
-                a.out_status[row] = TMS_ROW_OK;
-                if (a.out_keep) a.out_keep[row] = keep;
-            }
-            return;
+        whole = !(keep >= 2 && rank < keep - 1);
+        if (leader && !whole && t == 0) {
+            a.out_tokens[row] = tok;
+            a.out_status[row] = TMS_ROW_OK;
+            if (a.out_keep) a.out_keep[row] = keep;
         }
-        whole = true;
     }
-    if (!whole) return;
+    if (!leader) return;
+    if (shared && R.slot >= 0) {
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
+        lds_sync();
+        if (t == 0) __hip_atomic_store(&a.topp_locks[R.slot], 0u, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    if (inf) write_row_error(a, row, TMS_ROW_NONFINITE);
+    if (inf || !whole) return;
     lds_sync();
     if (t >= kBlock) return;
     [[clang::always_inline]] dense_inline<T>(a, row, L.u.d);

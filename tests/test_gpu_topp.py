@@ -147,3 +147,36 @@ def test_more_penalised_ids_than_a_record_holds(ctx, orc, high):
     mask = np.packbits(allowed, axis=1, bitorder="little").view(np.uint32)
     p = params_array(B, top_k=0, temperature=1.0, top_p=0.9, repeat_penalty=1.1, repeat_last_n=4000, seed=np.arange(B))
     check(run_gpu(ctx, x, p, recent=recent, mask=mask), orc.sample_batch(x, p, recent=recent, mask=mask))
+
+
+@pytest.mark.parametrize("dense", [20, 270])
+def test_slots_of_a_large_batch(ctx, orc, dense):
+    """A batch of more rows than slots: the rows left to the kernel have a slot
+    each, with helpers, or share them."""
+    B, V = 320, 9001
+    rng = np.random.default_rng(dense)
+    x, wide = _rows(rng, B, V, "bf16", 1.5)
+    p = _mixed(B, 3)
+    p["greedy"] = 1
+    p["greedy"][rng.choice(B, dense, replace=False)] = 0
+    want = orc.sample_batch(wide, p)
+    for _ in range(2):   # (the second on the locks that the first left)
+        check(run_gpu(ctx, x, p, dtype="bf16"), want)
+
+
+def test_workspace_of_large_contexts():
+    """Records are for 256 rows and 262144 ids at most: past them a row and an
+    id cost what the other regions take."""
+    from tensormark_amd import Sampler
+
+    def size(B, V):
+        s = Sampler(max_batch=B, max_vocab=V)
+        try:
+            return s.lib.tms_workspace_bytes(s.handle)
+        finally:
+            s.close()
+
+    row = (size(512, 32000) - size(256, 32000)) / 256      # lists, statistics, history lists
+    assert row < 128 * 1024, row
+    ids = (size(64, 524288) - size(64, 262144)) / 64 / 262144
+    assert ids < 17.0, ids                                   # the whole-row region's 16 bytes an id
