@@ -72,6 +72,11 @@ struct HistArgs {
     float* ov_vals;            // [B][kHistMax]
 };
 
+// Words of the breaker bits: brk_bits reads a position's word and the next,
+// up to position dn (a match that reaches the window's start).
+constexpr int kBrkWords = kDryMax / 32 + 2;
+static_assert((kDryMax >> 5) + 1 < kBrkWords, "brk_bits at the largest window's end");
+
 struct HistLds {
     uint32_t key[kHSlots];     // id + 1; 0 = empty (before the table: DRY's window past kHStage)
     uint32_t info[kHSlots];    // kHCount | kHDry | kHBan
@@ -81,7 +86,7 @@ struct HistLds {
     int32_t tslot[kHBlock];    // DRY: one tile of target slots, in position order
     float tsub[kHBlock];       //      and what each takes off: multiplier * base^(L - allowed_length)
     uint16_t dlen[kDryMax];    // DRY: the match length at each window position
-    uint32_t dbrk[kDryMax / 32 + 1];   // DRY: staged window positions holding a breaker
+    uint32_t dbrk[kBrkWords];  // DRY: staged window positions holding a breaker
     int wave_i[kHBlock / 64];
     int flag;                  // overflow
 };
@@ -158,7 +163,7 @@ __device__ __forceinline__ bool dry_eq(const int32_t* r, const uint32_t* brk, in
     return r[a] == r[b] && !((brk[a >> 5] >> (a & 31)) & 1u) && !((brk[b >> 5] >> (b & 31)) & 1u);
 }
 
-// The breaker bits of positions j .. j + 7, from bit 0.
+// The breaker bits of positions j .. j + 7, from bit 0 (j at most kDryMax).
 __device__ __forceinline__ uint32_t brk_bits(const uint32_t* brk, int j) {
     return (uint32_t)((((uint64_t)brk[(j >> 5) + 1] << 32) | brk[j >> 5]) >> (j & 31));
 }
@@ -220,7 +225,7 @@ __device__ void dry_lengths(const int32_t* r, int dn, HistLds& L) {
 // that many ids in one go, the ids and their breaker bits are read from
 // memory once, and DRY's terms are formed where their positions are listed,
 // so that an entry's subtractions wait on no load.  B = 16, 1024 ids, V =
-// 128256 bf16, n-gram ban and DRY: 17 us (256 threads, each pass reading
+// 128256 fp32, n-gram ban and DRY: 17 us (256 threads, each pass reading
 // the history again and an entry its exponents' scales one by one: 35).
 template <typename T>
 __global__ __launch_bounds__(kHBlock) void history_kernel(HistArgs a) {
@@ -253,7 +258,7 @@ __global__ __launch_bounds__(kHBlock) void history_kernel(HistArgs a) {
     const bool big = dn > kHStage;
     int32_t* r = big ? (int32_t*)L.key : L.win;
     if (dry_on) {
-        for (int i = t; i <= kDryMax / 32; i += kHBlock) L.dbrk[i] = 0u;
+        for (int i = t; i < kBrkWords; i += kHBlock) L.dbrk[i] = 0u;
         lds_sync();
     }
     for (int j = t; j < max(ns, dn); j += kHBlock) {

@@ -363,6 +363,24 @@ def test_history_window_edges(sampler, orc, n, last_n):
     check(g, want, 8)
 
 
+@pytest.mark.parametrize("n,match", [(33, 8), (33, 16), (1024, 56), (4096, 8), (4097, 64), (8192, 1), (8192, 7),
+                                     (8192, 8), (8192, 56), (8192, 63), (8192, 64), (8192, 72)])
+def test_dry_match_reaches_the_windows_start(sampler, orc, n, match):
+    """The window begins with the `match` ids that it ends with: their
+    comparison, eight positions a round, ends at the window's start."""
+    V = 20000
+    rng = np.random.default_rng(n + match)
+    recent = np.stack([rng.choice(V, n, replace=False) for _ in range(4)])
+    recent[:, :match] = recent[:, n - match:]
+    x = rng.normal(0, 1, (4, V)).astype(np.float32)
+    x[np.arange(4), recent[:, match]] += 30.0
+    p = params_array(4, temperature=0.8, top_k=40, top_p=0.95, seed=np.arange(4))
+    h = make_history(4, dry_multiplier=0.5, dry_base=1.1, dry_allowed_length=1, dry_penalty_last_n=n)
+    breaker = np.zeros(V, np.uint8)
+    got = _run(sampler, x, p, recent=recent, history=h, breaker=breaker, topk_cap=5)
+    check(got, orc.sample_batch(x, p, recent=recent, history=h, dry_breaker=breaker, topk_cap=5), 5)
+
+
 @pytest.mark.parametrize("n", [7, 8, 11, 12, 300, 1500])
 @pytest.mark.parametrize("pre_pass", [False, True])
 def test_long_repetition_chains(sampler, orc, n, pre_pass):
