@@ -130,11 +130,24 @@ __device__ __forceinline__ double uni(double v) {
     return __longlong_as_double((long long)((uint64_t)(uint32_t)uni((int)(u >> 32)) << 32 | (uint32_t)uni((int)u)));
 }
 
-// Where threads meet after a branch on thread 0 inside a loop that holds
-// barriers.  The compiler may otherwise merge the branch with a later one, and
-// take the other threads round the loop, and through its barriers, without
-// thread 0.  (A convergent no-op.)
-__device__ __forceinline__ void join() { __builtin_amdgcn_wave_barrier(); }
+// f() in thread 0, and every thread's value of f().  Every branch on thread 0
+// in this file is one of these: where two of them meet around a loop's backedge
+// with no barrier between, the compiler may otherwise merge them, and take the
+// other threads round the loop, and through its barriers, without thread 0.
+// (The wave barrier is a convergent no-op.)
+template <typename F>
+__device__ __forceinline__ void once(F&& f) {
+    if (threadIdx.x == 0) f();
+    __builtin_amdgcn_wave_barrier();
+}
+template <typename F>
+__device__ __forceinline__ uint32_t from_first(int& word, F&& f) {
+    once([&] { word = (int)f(); });
+    lds_sync();
+    const uint32_t v = (uint32_t)uni(word);
+    lds_sync();
+    return v;
+}
 
 __device__ __forceinline__ int excl_i(int v, int& total, Lds& L) {
     const int w = threadIdx.x >> 6;
@@ -203,6 +216,14 @@ __device__ __forceinline__ int block_min(int v, Lds& L) {   // v >= 0
     for (int i = 1; i < kW; ++i) r = min(r, L.wi[i]);
     lds_sync();
     return uni(r);
+}
+
+__device__ __forceinline__ void write_row(const KArgs& a, int row, int tok, int keep) {
+    once([&] {
+        a.out_tokens[row] = tok;
+        a.out_status[row] = TMS_ROW_OK;
+        if (a.out_keep) a.out_keep[row] = keep;
+    });
 }
 
 // put(i, v, id) for the entries i in [0, m) of the buckets [j0, j1] of nI
@@ -445,8 +466,7 @@ __device__ __forceinline__ void record(const KArgs& a, const Row& R, const tms_r
     for (int u = 0; u < 2; ++u) place(jo[u], lo[u]);
     lds_sync();
     for (int i = t; i < (total + 3) / 4; i += kT) st_agent(&rec[kHistId + i], ((const uint64_t*)H.ids)[i]);
-    if (t == 0) st_agent(&rec[kHistHead], (uint64_t)(lost ? 0 : 1) << 32 | __float_as_uint(lmax));
-    join();
+    once([&] { st_agent(&rec[kHistHead], (uint64_t)(lost ? 0 : 1) << 32 | __float_as_uint(lmax)); });
 }
 
 // The row, as every workgroup of it sees it before its records are read.
@@ -480,7 +500,7 @@ __device__ __forceinline__ bool plan(const KArgs& a, Row& R, Lds& L) {
     const int t = threadIdx.x;
     const uint64_t* rec = a.hist + (int64_t)R.slot * R.S * R.words;
     if (t < a.S) L.head[t] = ld_agent(&rec[(int64_t)t * R.words + kHistHead]);
-    if (t == 0) L.lost = 0;
+    once([&] { L.lost = 0; });
     lds_sync();
     float mx = -__builtin_huge_valf();
     for (int c = 0; c < a.S; ++c) mx = fmaxf(mx, __uint_as_float((uint32_t)L.head[c]));
@@ -773,7 +793,7 @@ __device__ __forceinline__ int select(const KArgs& a, const tms_row_params& P, c
     int pick = 0;
     if (keep >= 2) {
         // the sum over the kept prefix: the prefix at rank keep - 1
-        if (t == 0) L.misc[1] = 0;
+        once([&] { L.misc[1] = 0; });
         lds_sync();
 #pragma unroll
         for (int s = 0; s < kSelPer; ++s)
@@ -823,11 +843,7 @@ __device__ __forceinline__ int select(const KArgs& a, const tms_row_params& P, c
         if (probs) probs[i] = have ? (float)(exp((double)ckey_val(k) - mxd) / z) : 0.0f;
     }
     if (exact) return SEL_EXACT;
-    if (t == 0) {
-        a.out_tokens[R.row] = tok;
-        a.out_status[R.row] = TMS_ROW_OK;
-        if (a.out_keep) a.out_keep[R.row] = keep;
-    }
+    write_row(a, R.row, tok, keep);
     return SEL_DONE;
 }
 
@@ -1027,11 +1043,10 @@ __device__ __forceinline__ void emit(const Row& R, int n, double base, bool firs
     int nraw;
     int at = excl_i(__popc(rawm), nraw, L);
     if (nraw > kToppRawMax) {
-        if (t == 0) st_agent(&items[0], ~(uint64_t)0);
-        join();
+        once([&] { st_agent(&items[0], ~(uint64_t)0); });
         return;
     }
-    if (t == 0) L.se[0] = second && s0 * lo_f >= 0.5 ? -1 : expo(s0 * lo_f);
+    once([&] { L.se[0] = second && s0 * lo_f >= 0.5 ? -1 : expo(s0 * lo_f); });
     if (rawm) {
         double s = s0;
 #pragma unroll 1
@@ -1068,18 +1083,16 @@ __device__ __forceinline__ void emit(const Row& R, int n, double base, bool firs
             L.sw[k & 1][w][1] = f.a1;
         }
         lds_sync();
-        if (t == 0) {
+        once([&] {
             SeqFn g{0, 0};
             for (int q = 0; q < kW; ++q) g = then(g, SeqFn{L.sw[k & 1][q][0], L.sw[k & 1][q][1]});
             uint64_t* q = items + 1 + 3 * (2 * k);
             st_agent(&q[0], lo < hi ? (uint64_t)(L.se[k] + 2048) << 20 | (uint64_t)lo : (uint64_t)2 << 40);
             st_agent(&q[1], (uint64_t)g.a0);
             st_agent(&q[2], (uint64_t)g.a1);
-        }
-        join();
+        });
     }
-    if (t == 0) st_agent(&items[0], (uint64_t)(2 * nraw + 1));
-    join();
+    once([&] { st_agent(&items[0], (uint64_t)(2 * nraw + 1)); });
 }
 
 // Composes the row's items in order.  res[0]: 0 the sum never reached the
@@ -1088,7 +1101,6 @@ __device__ __forceinline__ void emit(const Row& R, int n, double base, bool firs
 // res[1], 3 the items do not fit together.
 __device__ __forceinline__ void compose(const uint64_t* items, int nr, bool second, Lds& L) {
     const int t = threadIdx.x;
-    if (t == 0) L.misc[0] = 0;
     int c = 0;
     if (t < nr) {
         const uint64_t h = ld_agent(&items[(int64_t)t * kToppItemWords]);
@@ -1097,10 +1109,10 @@ __device__ __forceinline__ void compose(const uint64_t* items, int nr, bool seco
     int total;
     const int at = excl_i(c, total, L);
     if (t < nr) L.off[t] = at;
-    if (t == 0) L.off[nr] = total;
+    once([&] { L.off[nr] = total; });
     lds_sync();
     if (total > kItems || total < 0) {
-        if (t == 0) L.res[0] = 3;
+        once([&] { L.res[0] = 3; });
         lds_sync();
         return;
     }
@@ -1159,12 +1171,12 @@ __device__ __forceinline__ void compose(const uint64_t* items, int nr, bool seco
         }
         const double s = value();
         if (r0 == 0) r1 = (int64_t)__double_as_longlong(s);
-        if (t == 0) {
+        once([&] {
             L.res[0] = r0;
             L.res[1] = r1;
             L.res[2] = r2;
             L.res[3] = r3;
-        }
+        });
     }
     lds_sync();
 }
@@ -1204,28 +1216,20 @@ __device__ __forceinline__ int reach_one(int n, int lo, int64_t S0, Lds& L) {
     return block_min(hit, L);
 }
 
-// Thread 0's value.
-__device__ __forceinline__ uint32_t bcast(uint32_t v, Lds& L) {
-    if (threadIdx.x == 0) L.misc[7] = (int)v;
-    lds_sync();
-    v = (uint32_t)uni(L.misc[7]);
-    lds_sync();
-    return v;
-}
-
 __device__ __forceinline__ uint32_t add_agent(uint32_t* p, uint32_t v) {
     return __hip_atomic_fetch_add(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
 // Thread 0 polls until *p >= want (bounded); the result is uniform.
 __device__ __forceinline__ bool wait_ge(const uint32_t* p, uint32_t want, int polls, Lds& L) {
-    uint32_t ok = 0;
-    if (threadIdx.x == 0)
+    return from_first(L.misc[7], [&] {
+        uint32_t ok = 0;
         for (int i = 0; i < polls && !ok; ++i) {
             ok = ld_agent(p) >= want ? 1u : 0u;
             if (!ok) __builtin_amdgcn_s_sleep(2);
         }
-    return bcast(ok, L) != 0;
+        return ok;
+    }) != 0;
 }
 
 // The kept prefix of a top_p = 1 row (leader: the row's first workgroup), or
@@ -1247,11 +1251,10 @@ __device__ __forceinline__ int exact_keep(const KArgs& a, const Row& R, bool lea
     auto begin = [&](int r) { return range_begin(r * Q, L); };
     auto end = [&](int r) { return r + 1 < nr ? range_begin((r + 1) * Q, L) : kHistBuckets - 1; };
     auto take = [&](int r) {   // a range's second pass, unless another workgroup has it
-        uint32_t got = 0;
-        if (t == 0)
-            got = !((__hip_atomic_fetch_or((unsigned long long*)&ctl[kCtlTaken], 1ull << r, __ATOMIC_RELAXED,
-                                           __HIP_MEMORY_SCOPE_AGENT) >> r) & 1ull);
-        return bcast(got, L) != 0;
+        return from_first(L.misc[7], [&] {
+            return (uint32_t)!((__hip_atomic_fetch_or((unsigned long long*)&ctl[kCtlTaken], 1ull << r, __ATOMIC_RELAXED,
+                                                      __HIP_MEMORY_SCOPE_AGENT) >> r) & 1ull);
+        }) != 0;
     };
     // Stages (one place does a range's work): 0 the ranges this workgroup
     // claims, for z; 1 the same ranges again, the one in LDS first, for the
@@ -1266,14 +1269,10 @@ __device__ __forceinline__ int exact_keep(const KArgs& a, const Row& R, bool lea
     for (;;) {
         int r = -1;
         if (stage == CLAIM) {
-            uint32_t q = 0;
-            if (t == 0) q = add_agent(&ctl[kCtlClaim], 1u);
-            join();
-            q = bcast(q, L);
+            const uint32_t q = from_first(L.misc[7], [&] { return add_agent(&ctl[kCtlClaim], 1u); });
             if (q < (uint32_t)nr) {
                 r = (int)q;
-                if (t == 0) L.mine[nmine] = r;
-                join();
+                once([&] { L.mine[nmine] = r; });
                 ++nmine;
             } else {
                 uint64_t zb = 0;
@@ -1282,15 +1281,14 @@ __device__ __forceinline__ int exact_keep(const KArgs& a, const Row& R, bool lea
                     const bool in = wait_ge(&ctl[kCtlDone1], (uint32_t)nr, kPollCap, L);
                     if (in) compose(items, nr, false, L);
                     zb = in && uni((int)L.res[0]) == 0 ? (uint64_t)readlane_i64(L.res[1], 0) : 0ull;
-                    if (t == 0) {
+                    once([&] {
                         st_agent((uint64_t*)&ctl[kCtlZ], zb);
                         __builtin_amdgcn_s_waitcnt(0);
                         st_agent(&ctl[kCtlPhase], 1u);
-                    }
-                    join();
+                    });
                 } else {
                     if (nmine == 0 || !wait_ge(&ctl[kCtlPhase], 1u, 1 << 12, L)) return -1;
-                    if (t == 0) L.res[1] = (int64_t)ld_agent((uint64_t*)&ctl[kCtlZ]);
+                    once([&] { L.res[1] = (int64_t)ld_agent((uint64_t*)&ctl[kCtlZ]); });
                     lds_sync();
                     zb = (uint64_t)readlane_i64(L.res[1], 0);
                 }
@@ -1311,11 +1309,11 @@ __device__ __forceinline__ int exact_keep(const KArgs& a, const Row& R, bool lea
                 // sums reach 1.0 in one of them, if at all.
                 if (!(have && divided && uni(L.pm[end(held)]) > z * (1.0 - 1e-6))) return -1;
                 if (!wait_ge(&ctl[kCtlPhase], 2u, 1 << 12, L)) return -1;
-                if (t == 0) {
+                once([&] {
                     L.res[1] = (int64_t)ld_agent((uint64_t*)&ctl[kCtlSum]);
                     L.res[2] = (int64_t)ld_agent(&ctl[kCtlReach]) - 1;
                     L.res[3] = (int64_t)ld_agent(&ctl[kCtlAt]);
-                }
+                });
                 lds_sync();
                 S1 = L.res[1];
                 at = uni((int)L.res[3]);
@@ -1342,23 +1340,18 @@ __device__ __forceinline__ int exact_keep(const KArgs& a, const Row& R, bool lea
                 r = uni((int)L.res[2]);
                 at = uni((int)L.res[3]);
                 lds_sync();
-                if (t == 0) {
+                once([&] {
                     st_agent((uint64_t*)&ctl[kCtlSum], (uint64_t)S1);
                     st_agent(&ctl[kCtlAt], (uint32_t)at);
                     st_agent(&ctl[kCtlReach], kind == 2 && held != r ? (uint32_t)r + 1u : 0u);
                     __builtin_amdgcn_s_waitcnt(0);
                     st_agent(&ctl[kCtlPhase], 2u);
-                }
-                join();
+                });
                 if (kind == 3) return -1;
                 if (kind == 0) return R.K;
                 if (kind == 1) return L.pc[begin(r)] + at + 1;
-                if (held != r && wait_ge(&ctl[kCtlKeep], 1u, kGrace, L)) {
-                    uint32_t q = 0;
-                    if (t == 0) q = ld_agent(&ctl[kCtlKeep]);
-                    join();
-                    return (int)bcast(q, L);
-                }
+                if (held != r && wait_ge(&ctl[kCtlKeep], 1u, kGrace, L))
+                    return (int)from_first(L.misc[7], [&] { return ld_agent(&ctl[kCtlKeep]); });
                 stage = REACH;
             }
         }
@@ -1379,21 +1372,18 @@ __device__ __forceinline__ int exact_keep(const KArgs& a, const Row& R, bool lea
             if (stage == REACH) {
                 const int i = reach_one(held_n, at, S1, L);
                 const int keep = i == kNone ? -1 : L.pc[j0] + i + 1;
-                if (!leader && t == 0 && keep > 0) st_agent(&ctl[kCtlKeep], (uint32_t)keep);
-                join();
+                if (!leader && keep > 0) once([&] { st_agent(&ctl[kCtlKeep], (uint32_t)keep); });
                 return keep;
             }
             emit(R, held_n, second ? L.pm[j0] / z : L.pm[j0], r == 0, second, out, L);
         } else {
             if (stage == REACH) return -1;
-            if (t == 0) st_agent(&out[0], ~(uint64_t)0);
-            join();
+            once([&] { st_agent(&out[0], ~(uint64_t)0); });
         }
         // the items are stored; then the range's done count
         __builtin_amdgcn_s_waitcnt(0);   // this wave's stores
         lds_sync();
-        if (t == 0) add_agent(&ctl[second ? kCtlDone2 : kCtlDone1], 1u);
-        join();
+        once([&] { add_agent(&ctl[second ? kCtlDone2 : kCtlDone1], 1u); });
     }
 }
 
@@ -1432,16 +1422,12 @@ template <typename T>
 __device__ __forceinline__ void records(const KArgs& a, const Row& R, const tms_row_params& P, uint32_t* ctl, Lds& L) {
     const int t = threadIdx.x;
     for (;;) {
-        uint32_t c = 0;
-        if (t == 0) c = add_agent(&ctl[kCtlChunk], 1u);
-        join();
-        c = bcast(c, L);
+        const uint32_t c = from_first(L.misc[7], [&] { return add_agent(&ctl[kCtlChunk], 1u); });
         if (c >= (uint32_t)R.S) break;
         record<T>(a, R, P, (int)c, L);
         __builtin_amdgcn_s_waitcnt(0);   // this wave's stores
         lds_sync();
-        if (t == 0) add_agent(&ctl[kCtlChunks], 1u);
-        join();
+        once([&] { add_agent(&ctl[kCtlChunks], 1u); });
     }
 }
 
@@ -1475,12 +1461,7 @@ __global__ __launch_bounds__(kT) void topp_kernel(KArgs a, int B) {
     // state words and parameters were written before this launch
     Row R;
     R.slot = g % n;   // pick_row's row
-    if (shared) {
-        if (t == 0) L.misc[6] = take_dense_slot(a.topp_locks, a.topp_slots, g);
-        lds_sync();
-        R.slot = uni(L.misc[6]);
-        lds_sync();
-    }
+    if (shared) R.slot = (int)from_first(L.misc[7], [&] { return take_dense_slot(a.topp_locks, a.topp_slots, g); });
     bool whole = R.slot < 0;
     int how = SEL_WHOLE, tok = -1, rank = 0;
     for (int turn = leader ? 1 : 0; turn < 2 && !whole; ++turn) {
@@ -1510,17 +1491,13 @@ __global__ __launch_bounds__(kT) void topp_kernel(KArgs a, int B) {
     if (!whole && !inf && (!leader || how == SEL_EXACT)) {
         const int keep = exact_keep<T>(a, R, leader, L);
         whole = !(keep >= 2 && rank < keep - 1);
-        if (leader && !whole && t == 0) {
-            a.out_tokens[row] = tok;
-            a.out_status[row] = TMS_ROW_OK;
-            if (a.out_keep) a.out_keep[row] = keep;
-        }
+        if (leader && !whole) write_row(a, row, tok, keep);
     }
     if (!leader) return;
     if (shared && R.slot >= 0) {
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
         lds_sync();
-        if (t == 0) __hip_atomic_store(&a.topp_locks[R.slot], 0u, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
+        once([&] { __hip_atomic_store(&a.topp_locks[R.slot], 0u, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT); });
     }
     if (inf) write_row_error(a, row, TMS_ROW_NONFINITE);
     if (inf || !whole) return;

@@ -108,3 +108,14 @@ def test_row_kind_constants_and_sparse_mask_hint():
     bits[2, :2049] = True          # one row past it
     assert not sampler.mask_is_sparse(workloads.pack_bits(bits))
     assert sampler.mask_is_sparse(workloads.cfg3()["mask"])
+
+
+def test_branches_on_thread_zero_go_through_one_helper():
+    """tms_topp.hip: the compiler merged two branches on thread 0 around a
+    loop's backedge and took the other threads through the loop's barriers
+    without it.  Such branches are `once` and `from_first`, which cannot be
+    merged; a bare one is not written there."""
+    src = open(os.path.join(ROOT, "tensormark_amd", "csrc", "tms_topp.hip")).read()
+    code = re.sub(r"//[^\n]*", "", src)
+    assert len(re.findall(r"\bthreadIdx\.x\s*==\s*0", code)) == 1
+    assert not re.findall(r"\bt\s*==\s*0\b|!\s*t\b|!\s*threadIdx", code)
