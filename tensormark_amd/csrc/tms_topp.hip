@@ -25,7 +25,7 @@
 // functions, leaving out the few entries at which s may change its binade;
 // the row's first workgroup composes the ranges.  Twice: z, then the sums of
 // pr / z.  The serial loop that this replaces took about 290 ns an entry: a
-// call of B = 32, V = 256000 fp16 with six such rows 79.0 ms, now 0.26.
+// call of B = 32, V = 256000 fp16 with six such rows 79.0 ms, now 0.2.
 //
 // Bound by latency, not by bytes: a nucleus row of V = 128256 takes 50.7 us
 // (2294 sorted whole) as a chain of the general kernel's lists (10), the
@@ -1016,27 +1016,19 @@ __device__ __forceinline__ void emit(const Row& R, int n, double base, bool firs
     for (int j = 0; j < kPer; ++j) s0 += L.u.x[t * kPer + j];
     s0 = base + excl_d(s0, tot, L);
     const double lo_f = 1.0 - 4.0 * R.rel, hi_f = 1.0 + 4.0 * R.rel;
-    // Per entry, once: whether it is raw, the whole part of its increment and
-    // how the rest rounds.
-    uint32_t rawm = 0, up = 0, tie = 0;
-    int64_t fl[kPer];
+    uint32_t rawm = 0;   // the raw entries
     {
         double s = s0;
 #pragma unroll
         for (int j = 0; j < kPer; ++j) {
             const int i = t * kPer + j;
-            const double lo = s * lo_f, x = L.u.x[i];
-            s += x;
+            const double lo = s * lo_f;
+            s += L.u.x[i];
             const bool last = second && lo >= 0.5;
             bool raw = !(lo > 0.0) || expo(lo) != expo(s * hi_f);
             if (last) raw = false;
             if (first && i == 0) raw = true;
             if (raw && i < n) rawm |= 1u << j;
-            const int e = last ? -1 : expo(lo);
-            const double y = raw || i >= n ? 0.0 : x * pow2(52 - e), m = floor(y);
-            fl[j] = (int64_t)m;
-            up |= y - m > 0.5 ? 1u << j : 0u;
-            tie |= y - m == 0.5 ? 1u << j : 0u;
             __builtin_amdgcn_sched_barrier(0);
         }
     }
@@ -1066,17 +1058,22 @@ __device__ __forceinline__ void emit(const Row& R, int n, double base, bool firs
     for (int k = 0; k <= nraw; ++k) {
         const int lo = k ? uni(L.raw[k - 1]) + 1 : 0, hi = k < nraw ? uni(L.raw[k]) : n;
         SeqFn f{0, 0};
+        // A wave's entries fall in few runs; the others it leaves out.  (An
+        // entry's function is formed in its run, of whose binade it is, and not
+        // kept from one run to the next: 22 registers.)
+        const int w0 = (t & ~63) * kPer;
+        if (hi > w0 && lo < w0 + 64 * kPer) {
+            const double scale = pow2(52 - uni(L.se[k]));
 #pragma unroll
-        for (int j = 0; j < kPer; ++j) {
-            const int i = t * kPer + j;
-            const int64_t m = fl[j], odd = m & 1, u = (up >> j) & 1u;
-            const bool ti = (tie >> j) & 1u;
-            if (i >= lo && i < hi) f = then(f, SeqFn{m + (ti ? odd : u), m + (ti ? 1 - odd : u)});
-        }
+            for (int j = 0; j < kPer; ++j) {
+                const int i = t * kPer + j;
+                if (i >= lo && i < hi) f = then(f, seq_fn(L.u.x[i] * scale));
+            }
 #pragma unroll
-        for (int d = 1; d < 64; d <<= 1) {
-            const SeqFn o = shfl_down(f, d);
-            if ((lane & (2 * d - 1)) == 0) f = then(f, o);
+            for (int d = 1; d < 64; d <<= 1) {
+                const SeqFn o = shfl_down(f, d);
+                if ((lane & (2 * d - 1)) == 0) f = then(f, o);
+            }
         }
         if (lane == 0) {
             L.sw[k & 1][w][0] = f.a0;
@@ -1315,7 +1312,7 @@ __device__ __forceinline__ int exact_keep(const KArgs& a, const Row& R, bool lea
                     L.res[3] = (int64_t)ld_agent(&ctl[kCtlAt]);
                 });
                 lds_sync();
-                S1 = L.res[1];
+                S1 = readlane_i64(L.res[1], 0);
                 at = uni((int)L.res[3]);
                 const bool here = uni((int)L.res[2]) == held;
                 lds_sync();
@@ -1336,7 +1333,7 @@ __device__ __forceinline__ int exact_keep(const KArgs& a, const Row& R, bool lea
                 if (!wait_ge(&ctl[kCtlDone2], (uint32_t)nr, kPollCap, L)) return -1;
                 compose(items, nr, true, L);
                 const int kind = uni((int)L.res[0]);
-                S1 = L.res[1];
+                S1 = readlane_i64(L.res[1], 0);
                 r = uni((int)L.res[2]);
                 at = uni((int)L.res[3]);
                 lds_sync();
