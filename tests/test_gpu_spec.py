@@ -76,9 +76,8 @@ def test_spec_cfg4_full_size(orc, sampler):
 
 def test_spec_caller_draws_and_dtypes(orc, sampler):
     rng = np.random.default_rng(41)
-    # 16-byte aligned rows (V a multiple of 4 for f32, 8 for f16/bf16) take the
-    # chunked statistics (4096 ids a chunk, the last one ragged); the others
-    # the per-row kernel.
+    # Whole 16-byte vectors a row (V a multiple of 4 for f32, 8 for f16/bf16)
+    # and rows at any element's address; one part a row and several.
     for dtype, V, k in [("f32", 1000, 3), ("f16", 4096, 5), ("bf16", 777, 16), ("f32", 5, 1),
                         ("f32", 50000, 2), ("bf16", 10000, 4), ("f16", 12296, 3)]:
         B = 6
@@ -171,23 +170,27 @@ def test_spec_back_to_back_different_batches(orc, sampler):
         check_spec(orc, gpu, c["target"], c["draft"], c["tokens"], c["params"], words)
 
 
-@pytest.mark.parametrize("B,V", [(24, 140000), (4, 262144)])
-def test_spec_resolve_ticket_form(orc, sampler, B, V):
-    """Resolve grids that are not resident at once (24 sequences x 64 parts)
-    and part runs past 16 ids a thread (V = 262144: 4,096 ids a part) take
-    the ticket form, whose last arriver recomputes the threshold's part;
-    config 4 itself takes the waiting form.  Rows this long also take the
-    two-pass statistics kernel."""
+@pytest.mark.parametrize("dtype", ["f32", "bf16"])
+@pytest.mark.parametrize("B,V", [(24, 140000), (4, 262144), (40, 140000), (2, 262145), (9, 300003)])
+def test_spec_resolve_forms(orc, sampler, dtype, B, V):
+    """The waiting resolve with 16 ids a thread (35 and 64 parts a sequence),
+    its grid resident at once or taking its places in order, and the ticket
+    form past 262144 ids, whose last arriver reads the threshold's part again,
+    in runs of more than 16 ids a thread."""
+    if V > 262144:
+        from tensormark_amd import Sampler
+
+        sampler = Sampler(max_batch=B, max_vocab=V)
     rng = np.random.default_rng(B)
     k = 2
-    target = rng.normal(0.0, 2.0, (B, k + 1, V)).astype(np.float32)
-    draft = (target[:, :k] + rng.normal(0.0, 0.5, (B, k, V))).astype(np.float32)
+    target = rng.standard_normal((B, k + 1, V), dtype=np.float32) * 2.0
+    draft = target[:, :k] + 0.5 * rng.standard_normal((B, k, V), dtype=np.float32)
     tokens = workloads.softmax_draws(rng, draft)
     params = params_array(B, temperature=1.0, top_k=0, top_p=1.0, seed=np.arange(B) + 3)
     params["temperature"] = rng.choice([0.8, 1.0], size=B)
-    gpu = run_spec(sampler, target, draft, tokens, params)
+    gpu = run_spec(sampler, target, draft, tokens, params, dtype=dtype)
     words = philox_words(orc, params, k)
-    check_spec(orc, gpu, target, draft, tokens, params, words)
+    check_spec(orc, gpu, target, draft, tokens, params, words, dtype)
     assert (gpu["status"] == 0).all()
 
 
