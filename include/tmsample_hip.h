@@ -532,6 +532,11 @@ int tms_debug_exp(const double* in, double* out, int n, int which, hipStream_t s
  * another's result before it forms that result itself (negative: the
  * default; 0: at once).  The answers do not depend on it. */
 int tms_debug_spec_polls(tms_context* ctx, int polls);
+/* How the last sampling call on this context, without the top-k promise or the
+ * sparse-mask hint, decided its first `batch` rows: 0 from the chunk lists, 1
+ * by buckets, 2 by the sums of top_p = 1, 3 over the whole row, 4 not at all
+ * (v / T overflowed).  For vocab <= 262144.  Synchronous. */
+int tms_debug_row_forms(tms_context* ctx, int batch, int32_t* forms);
 
 #ifdef __cplusplus
 }

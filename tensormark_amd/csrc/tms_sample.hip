@@ -42,6 +42,7 @@
 #include <algorithm>
 #include <atomic>
 #include <mutex>
+#include <vector>
 
 #include "tms_dense.h"
 #include "tms_select.h"
@@ -1603,6 +1604,16 @@ extern "C" int tms_sample_batch(tms_context* ctx, const tms_sample_args* a, hipS
     w.topp_call = ++ctx->topp_calls;
     w.topp_items = ctx->topp_items;
     return sample_launch(w, a, stream);
+}
+
+extern "C" int tms_debug_row_forms(tms_context* ctx, int batch, int32_t* forms) {
+    if (!ctx || !forms || batch <= 0 || batch > ctx->max_batch) return TMS_ERR_INVALID_ARG;
+    std::vector<uint32_t> ctl((size_t)batch * tms::kToppCtl);
+    if (hipDeviceSynchronize() != hipSuccess ||
+        hipMemcpy(ctl.data(), ctx->topp_ctl, ctl.size() * 4, hipMemcpyDeviceToHost) != hipSuccess)
+        return TMS_ERR_HIP;
+    for (int i = 0; i < batch; ++i) forms[i] = (int32_t)ctl[(size_t)i * tms::kToppCtl + tms::kToppForm];
+    return TMS_OK;
 }
 
 // ============================================= allocation-free entry point

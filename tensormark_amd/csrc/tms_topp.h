@@ -48,6 +48,11 @@ inline size_t topp_hist_words(size_t rows, int vocab) {
 }
 // Row states the general kernel leaves for the whole-vocabulary kernel.
 enum : uint32_t { TOPP_NONE = 0, TOPP_SELECT = 1, TOPP_WHOLE = 2 };
+// How that kernel decided a row (word kToppForm of the row's shared words): by
+// the buckets of the cut and the draw, by the composed sums of top_p = 1, or
+// by the full-row form.
+enum : uint32_t { TOPP_BY_BUCKETS = 1, TOPP_BY_SUMS = 2, TOPP_BY_ROW = 3, TOPP_NOT_FINITE = 4 };
+constexpr int kToppForm = 18;
 // u32 words per row shared by the workgroups of a row (zeroed by the general
 // kernel's merger): see tms_topp.hip.
 constexpr int kToppCtl = 64;

@@ -65,7 +65,7 @@ constexpr int kMaxSeg = 64;        // (interval, chunk) runs of a fetch
 constexpr int kGrace = 1 << 8;   // polls before the first workgroup takes over unclaimed ranges
 // Shared words of a row (u32 index; the general kernel zeroed them).
 enum { kCtlState = 0, kCtlClaim = 1, kCtlDone1 = 2, kCtlPhase = 3, kCtlDone2 = 4, kCtlTaken = 6, kCtlZ = 8,
-       kCtlSum = 10, kCtlAt = 12, kCtlReach = 13, kCtlKeep = 14, kCtlChunk = 16, kCtlChunks = 17 };
+       kCtlSum = 10, kCtlAt = 12, kCtlReach = 13, kCtlKeep = 14, kCtlChunk = 16, kCtlChunks = 17, kCtlForm = kToppForm };
 
 struct Lds {
     union {
@@ -1496,6 +1496,10 @@ __global__ __launch_bounds__(kT) void topp_kernel(KArgs a, int B) {
         lds_sync();
         once([&] { __hip_atomic_store(&a.topp_locks[R.slot], 0u, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT); });
     }
+    once([&] {
+        a.topp_ctl[(int64_t)row * kToppCtl + kCtlForm] =
+            whole ? TOPP_BY_ROW : inf ? TOPP_NOT_FINITE : how == SEL_EXACT ? TOPP_BY_SUMS : TOPP_BY_BUCKETS;
+    });
     if (inf) write_row_error(a, row, TMS_ROW_NONFINITE);
     if (inf || !whole) return;
     lds_sync();

@@ -42,6 +42,7 @@ EXPORTS = (
     "tms_debug_philox",
     "tms_debug_exp",
     "tms_debug_spec_polls",
+    "tms_debug_row_forms",
     "tms_host_repeat_penalty",
     "tms_host_no_repeat_ngram",
     "tms_host_dry",
@@ -258,6 +259,7 @@ def load_library(path: str = LIB_PATH) -> C.CDLL:
         lib.tms_debug_philox.argtypes = [C.c_void_p, C.c_void_p, C.c_int, C.c_void_p]
         lib.tms_debug_ordering.argtypes = [C.c_int, C.POINTER(C.c_int32)]
         lib.tms_workspace_reset.argtypes = [C.c_void_p, C.c_void_p]
+        lib.tms_debug_row_forms.argtypes = [C.c_void_p, C.c_int, C.POINTER(C.c_int32)]
         lib.tms_debug_spec_polls.argtypes = [C.c_void_p, C.c_int]
         lib.tms_debug_exp.argtypes = [C.c_void_p, C.c_void_p, C.c_int, C.c_int, C.c_void_p]
         fp, ip = C.POINTER(C.c_float), C.POINTER(C.c_int32)
