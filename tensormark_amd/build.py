@@ -38,9 +38,10 @@ HIPCC_FLAGS = [
 # result is broadcast at once, waiting out the round trip there.  The
 # whole-vocabulary kernel is many phases in one loop: constants hoisted out of
 # it would live through every phase, in scratch (44 bytes a lane; none without).
+# Its first four argument words come in registers.
 FILE_FLAGS = {
     "tms_wide.hip": ["-mllvm", "-amdgpu-atomic-optimizer-strategy=None"],
-    "tms_topp.hip": ["-mllvm", "-disable-machine-licm"],
+    "tms_topp.hip": ["-mllvm", "-disable-machine-licm", "-mllvm", "-amdgpu-kernarg-preload-count=4"],
 }
 
 BUILD_DIR = os.path.join(HERE, "_build")
