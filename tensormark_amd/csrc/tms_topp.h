@@ -14,8 +14,14 @@ namespace tms {
 //
 // Buckets run from the one holding the chunk's maximum downwards: 1023 x 1/25
 // spans 40.9, more than kSigSpan, so every entry that can change a sum has
-// one.  At 1/25 a bucket of a 256,000-id normal row holds at most about 1,700
-// entries, so a cut or a draw is settled by ordering a few thousand keys.
+// one.  The fullest bucket of a normal row holds about 0.016 V / d entries, d the
+// standard deviation of lg: 1,640 of 256,000 at d = 2.5.  So a cut and a draw
+// are settled by ordering a few thousand keys (kSel at most) where a row is not
+// flat.  Rows that took the full-row form, of 64 normal rows at top_p 0.9, 0.95
+// and 0.98: V = 256000 none or one at d >= 2.5, 3 to 5 at 2.0, 12 to 16 at 1.67,
+// 31 to 44 at 1.25; V = 128256 none at 1.67, up to 8 at 1.25, 4 to 11 at 1.0; V =
+// 32000 none at 0.5.  With top_p = 1 (kRange): V = 256000 none at 1.25, two at
+// 1.0; V = 128256 none at 0.75, seven at 0.5.
 constexpr int kHistBuckets = 1024;
 constexpr float kHistScale = 25.0f;
 constexpr int kHistExtra = 1024;        // penalised entries of a chunk, at most

@@ -25,12 +25,12 @@
 // functions, leaving out the few entries at which s may change its binade;
 // the row's first workgroup composes the ranges.  Twice: z, then the sums of
 // pr / z.  The serial loop that this replaces took about 290 ns an entry: a
-// call of B = 32, V = 256000 fp16 with six such rows 79.0 ms, now 0.2.
+// call of B = 32, V = 256000 fp16 with six such rows 79.0 ms, now 0.15.
 //
-// Bound by latency, not by bytes: a nucleus row of V = 128256 takes 50.7 us
+// Bound by latency, not by bytes: a nucleus row of V = 128256 takes 50.6 us
 // (2294 sorted whole) as a chain of the general kernel's lists (10), the
 // records (9: LDS atomics), the plan (7), the bucket search and fetch (7), the
-// ordering (4) and the sums and pick (5 to 14); 64 of them 71.8 us (3422).
+// ordering (4) and the sums and pick (5 to 14); 64 of them 72.2 us (3422).
 //
 // The first workgroups of the launch take a row each, the rest, up to one a CU
 // in all, help them.  A chunk or a range is claimed by an atomic counter, so no
@@ -836,6 +836,10 @@ __device__ __forceinline__ int select(const KArgs& a, const tms_row_params& P, c
     lds_sync();
     tok = uni(L.misc[2]);
     rank = pick;
+    // (A bucket's mass is added up in no fixed order, so z differs by some 2^-50
+    // of itself from call to call, and a probability by its last bit where that
+    // moves its rounding, about once in 10^7.  The decisions above do not depend
+    // on it: within the margin they are the full-row form's.)
     for (int i = t; i < cap; i += kT) {
         const bool have = i < R.n && i < R.K;
         const uint64_t k = have ? L.u.s.srt[i] : 0ull;
